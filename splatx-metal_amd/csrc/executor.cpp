@@ -111,8 +111,21 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
     if (!s) invalid("TrainStepExecutor", "null sync");
     if (s->rows < 0 || s->rows > e->rows) invalid("TrainStepExecutor", "sync rows out of [0, arena_rows]");
     const int rows = static_cast<int>(s->rows);
-    sxh_detail::canonicalize(e);  // rows in the caller's order, the pending update applied
+    if (up && !(e->permuted && rows >= e->perm_count)) {
+        sxh_detail::canonicalize(e);  // rows in the caller's order, the pending update applied
+    } else {
+        // a download puts each row in its caller's place as it packs it, and the arena keeps its order; an
+        // upload over every permuted row replaces them all, so they need not move back first
+        sxh_detail::flush_update(e);
+        if (up) {
+            e->permuted = false;
+            e->steps_since_exchange = 0;
+        }
+    }
     if (rows == 0) return;
+    // rows packed: with the arena in spatial order a row below `rows` may stand anywhere in the permuted part
+    const int n_pack = e->permuted ? std::max(rows, e->perm_count) : rows;
+    const int32_t* const place = e->permuted ? e->row_orig.p : nullptr;
     hipStream_t st = e->b->stream;
     for (int g = 0; g < 6; g++) {
         const int dim = e->dims[g];
@@ -124,9 +137,9 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
             const size_t n = static_cast<size_t>(rows) * dim;
             if (up) {
                 SXH_HIP(hipMemcpyAsync(e->staging.p, host[k], n * 4, hipMemcpyHostToDevice, st));
-                sxk::aos_to_soa(e->staging.p, dev[k]->p, rows, dim, e->rows, st);
+                sxk::rows_to_soa(e->staging.p, dev[k]->p, rows, dim, e->rows, st);
             } else {
-                sxk::soa_to_aos(dev[k]->p, e->staging.p, rows, dim, e->rows, st);
+                sxk::soa_to_rows(dev[k]->p, e->staging.p, n_pack, dim, e->rows, st, place, e->perm_count, rows);
                 SXH_HIP(hipMemcpyAsync(host[k], e->staging.p, n * 4, hipMemcpyDeviceToHost, st));
             }
             SXH_HIP(hipStreamSynchronize(st));  // staging is reused

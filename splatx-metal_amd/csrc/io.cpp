@@ -528,7 +528,7 @@ int32_t sxh_render_session_open(sxh_backend* b, const sxh_render_session_args* a
             for (int g = 0; g < 6; g++) {  // parameters only; the moments stay zero
                 if (e->dims[g] == 0) continue;
                 SXH_HIP(hipMemcpyAsync(e->staging.p, c.g[g].data(), c.g[g].size() * 4, hipMemcpyHostToDevice, s));
-                sxk::aos_to_soa(e->staging.p, e->p[g].p, static_cast<int>(c.count), e->dims[g], e->rows, s);
+                sxk::rows_to_soa(e->staging.p, e->p[g].p, static_cast<int>(c.count), e->dims[g], e->rows, s);
                 SXH_HIP(hipStreamSynchronize(s));
             }
         } catch (...) {

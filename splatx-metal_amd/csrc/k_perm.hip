@@ -7,11 +7,14 @@
 // live rows [0, count) in that order, with the maps between its internal rows and the caller's
 // (original) rows. Every result stays the caller's: depth first, the emit runs in original order (so
 // the stable depth sort's ties go by original row); index first, it runs in internal order and the
-// per-tile depth sort puts equal depths in original-row order; the MCMC noise is drawn by original row,
-// and every entry point that exchanges rows with the caller restores the original order first.
+// per-tile depth sort puts equal depths in original-row order; the MCMC noise is drawn by original row; a
+// download puts each row in its original place as it packs it, and every other entry point that exchanges
+// rows with the caller restores the original order first.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <stdexcept>
+#include <type_traits>
 
 #include "sx_step.h"
 
@@ -114,20 +117,76 @@ __global__ void __launch_bounds__(kBlock) k_morton(const float* __restrict__ m, 
     vals[i] = i;
 }
 
-// tmp[d * count + k] = col[d * R + src[k]] for the dim columns of one arena array, rows k < count
-__global__ void __launch_bounds__(kBlock) k_gather_rows(const float* __restrict__ col, size_t R, int dim, int count,
-                                                        const int32_t* __restrict__ src, float* __restrict__ tmp) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
-    const size_t r = static_cast<size_t>(src[k]);
-    for (int d = 0; d < dim; d++) tmp[(size_t)d * count + k] = col[d * R + r];
+// Rows between the arena's columns (SoA, stride R) and row-major arrays of DIM floats per row, a block of
+// ROWS rows through LDS: the columns are read or written 64 rows at a time (256-B runs) and the row-major
+// side element by element along each row, so both sides are coalesced also where the rows go to (dst) or
+// come from (src) other places: a whole row is one run of 4 DIM bytes. Bound: HBM, 8 B per element. At 1 M rows and
+// SH3 the 45-column group takes 0.104 ms to pack and 0.076 ms to unpack (3.5 and 4.7 TB/s), and the whole
+// permutation of parameters and moments (18 arrays, through a row-major copy) about 0.95 ms. Before, a thread
+// per row-major element touched the columns at a stride of DIM threads (an upload's and a download's kernels
+// 0.97 and 0.73 ms), and a permutation gathered single floats from 177 columns (3.06 ms).
+
+// aos[dst(k) * DIM + d] = soa[d * R + k] for rows k < n, dst(k) = dst_row[k] below n_perm, k at or past it
+// (k where dst_row is null); rows whose place is at or past n_out are left out.
+template <int DIM, int ROWS>
+__global__ void __launch_bounds__(kBlock) k_rows_pack(const float* __restrict__ soa, size_t R, int n,
+                                                      const int32_t* __restrict__ dst_row, int n_perm, int n_out,
+                                                      float* __restrict__ aos) {
+    constexpr int kPitch = DIM | 1;  // an odd pitch: no bank conflicts down a column
+    __shared__ float s_v[ROWS * kPitch];
+    __shared__ int32_t s_dst[ROWS];
+    const int k0 = blockIdx.x * ROWS;
+    const int m = min(ROWS, n - k0);
+    for (int q = threadIdx.x; q < ROWS; q += kBlock) s_dst[q] = (dst_row && k0 + q < n_perm) ? dst_row[k0 + q] : k0 + q;
+    const int r = threadIdx.x % ROWS;
+#pragma unroll
+    for (int d = threadIdx.x / ROWS; d < DIM; d += kBlock / ROWS)
+        if (r < m) s_v[r * kPitch + d] = soa[(size_t)d * R + k0 + r];
+    __syncthreads();
+#pragma unroll 4
+    for (int q = threadIdx.x; q < m * DIM; q += kBlock) {
+        const int row = q / DIM, d = q - row * DIM;
+        const int to = s_dst[row];
+        if (to < n_out) aos[(size_t)to * DIM + d] = s_v[row * kPitch + d];
+    }
 }
 
-__global__ void __launch_bounds__(kBlock) k_put_rows(const float* __restrict__ tmp, size_t R, int dim, int count,
-                                                     float* __restrict__ col) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= count) return;
-    for (int d = 0; d < dim; d++) col[d * R + k] = tmp[(size_t)d * count + k];
+// soa[d * R + k] = aos[src(k) * DIM + d] for rows k < n, src(k) = src_row[k] (k where src_row is null)
+template <int DIM, int ROWS>
+__global__ void __launch_bounds__(kBlock) k_rows_unpack(const float* __restrict__ aos, size_t R, int n,
+                                                        const int32_t* __restrict__ src_row, float* __restrict__ soa) {
+    constexpr int kPitch = DIM | 1;
+    __shared__ float s_v[ROWS * kPitch];
+    __shared__ int32_t s_src[ROWS];
+    const int k0 = blockIdx.x * ROWS;
+    const int m = min(ROWS, n - k0);
+    for (int q = threadIdx.x; q < m; q += kBlock) s_src[q] = src_row ? src_row[k0 + q] : k0 + q;
+    __syncthreads();
+#pragma unroll 4
+    for (int q = threadIdx.x; q < m * DIM; q += kBlock) {
+        const int row = q / DIM, d = q - row * DIM;
+        s_v[row * kPitch + d] = aos[(size_t)s_src[row] * DIM + d];
+    }
+    __syncthreads();
+    const int r = threadIdx.x % ROWS;
+#pragma unroll
+    for (int d = threadIdx.x / ROWS; d < DIM; d += kBlock / ROWS)
+        if (r < m) soa[(size_t)d * R + k0 + r] = s_v[r * kPitch + d];
+}
+
+// Calls f with the group's dimension as a compile-time constant (the six groups' dimensions at SH degrees 0-3)
+// and the rows of a block: 256 for the narrow groups, 64 where a row is 96 B and more (12 KB of LDS at most).
+template <class F>
+void with_dim(int dim, F&& f) {
+    switch (dim) {
+        case 1: f(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{}); return;
+        case 3: f(std::integral_constant<int, 3>{}, std::integral_constant<int, 256>{}); return;
+        case 4: f(std::integral_constant<int, 4>{}, std::integral_constant<int, 256>{}); return;
+        case 9: f(std::integral_constant<int, 9>{}, std::integral_constant<int, 256>{}); return;
+        case 24: f(std::integral_constant<int, 24>{}, std::integral_constant<int, 64>{}); return;
+        case 45: f(std::integral_constant<int, 45>{}, std::integral_constant<int, 64>{}); return;
+        default: throw std::invalid_argument("arena rows: no such group dimension");
+    }
 }
 
 // the maps of a permutation from the original order: internal row k holds original row src[k]
@@ -154,16 +213,30 @@ void arena_morton_keys(const Arena& A, int count, float* scratch, uint32_t* keys
 
 size_t arena_morton_scratch_floats(int count) { return 8 + 6 * static_cast<size_t>(grid_for(count)); }
 
+void soa_to_rows(const float* soa, float* aos, int n, int dim, int stride, hipStream_t s, const int32_t* dst_row,
+                 int n_perm, int n_out) {
+    if (n <= 0) return;
+    with_dim(dim, [&](auto D, auto B) {
+        hipLaunchKernelGGL((k_rows_pack<D(), B()>), dim3((n + B() - 1) / B()), dim3(kBlock), 0, s, soa,
+                           static_cast<size_t>(stride), n, dst_row, n_perm, n_out < 0 ? n : n_out, aos);
+    });
+}
+
+void rows_to_soa(const float* aos, float* soa, int n, int dim, int stride, hipStream_t s, const int32_t* src_row) {
+    if (n <= 0) return;
+    with_dim(dim, [&](auto D, auto B) {
+        hipLaunchKernelGGL((k_rows_unpack<D(), B()>), dim3((n + B() - 1) / B()), dim3(kBlock), 0, s, aos,
+                           static_cast<size_t>(stride), n, src_row, soa);
+    });
+}
+
 void arena_permute_rows(const Arena& A, const int dims[6], int count, const int32_t* src, float* tmp, hipStream_t s) {
     if (count <= 0) return;
-    const size_t R = static_cast<size_t>(A.rows);
     for (int g = 0; g < 6; g++) {
         if (dims[g] == 0) continue;
-        float* cols[3] = {A.p[g], A.m[g], A.v[g]};
-        for (float* col : cols) {
-            hipLaunchKernelGGL(k_gather_rows, dim3(grid_for(count)), dim3(kBlock), 0, s, col, R, dims[g], count, src,
-                               tmp);
-            hipLaunchKernelGGL(k_put_rows, dim3(grid_for(count)), dim3(kBlock), 0, s, tmp, R, dims[g], count, col);
+        for (float* col : {A.p[g], A.m[g], A.v[g]}) {
+            soa_to_rows(col, tmp, count, dims[g], A.rows, s);
+            rows_to_soa(tmp, col, count, dims[g], A.rows, s, src);
         }
     }
 }

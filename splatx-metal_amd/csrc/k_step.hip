@@ -886,22 +886,6 @@ __global__ void k_step_readback(StepReadback rb) {
     __hip_atomic_store(rb.seq_host, rb.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-__global__ void __launch_bounds__(kBlock) k_aos_to_soa(const float* __restrict__ aos, float* __restrict__ soa, int rows,
-                                                       int dim, int stride) {
-    const int64_t k = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    if (k >= (int64_t)rows * dim) return;
-    const int r = static_cast<int>(k / dim), d = static_cast<int>(k % dim);
-    soa[(size_t)d * stride + r] = aos[k];
-}
-
-__global__ void __launch_bounds__(kBlock) k_soa_to_aos(const float* __restrict__ soa, float* __restrict__ aos, int rows,
-                                                       int dim, int stride) {
-    const int64_t k = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    if (k >= (int64_t)rows * dim) return;
-    const int r = static_cast<int>(k / dim), d = static_cast<int>(k % dim);
-    aos[k] = soa[(size_t)d * stride + r];
-}
-
 } // namespace
 
 void step_preprocess(const StepConst& c, const Arena& A, float4* splats, int32_t* radii, int32_t* tiles,
@@ -1070,18 +1054,6 @@ void step_set_word(uint32_t* word, uint32_t value, hipStream_t s) {
 void step_readback(const StepReadback& rb, hipStream_t s) {
     if (!rb.host) return;
     hipLaunchKernelGGL(k_step_readback, dim3(1), dim3(1), 0, s, rb);
-}
-
-void aos_to_soa(const float* aos, float* soa, int rows, int dim, int stride, hipStream_t s) {
-    const int64_t n = (int64_t)rows * dim;
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_aos_to_soa, dim3(grid_for(n)), dim3(kBlock), 0, s, aos, soa, rows, dim, stride);
-}
-
-void soa_to_aos(const float* soa, float* aos, int rows, int dim, int stride, hipStream_t s) {
-    const int64_t n = (int64_t)rows * dim;
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_soa_to_aos, dim3(grid_for(n)), dim3(kBlock), 0, s, soa, aos, rows, dim, stride);
 }
 
 } // namespace sxk

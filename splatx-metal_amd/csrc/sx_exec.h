@@ -108,7 +108,7 @@ struct sxh_executor {
     // The live rows' order in HBM (sxh_exec_set_row_order, k_perm.hip). With `permuted`, internal row k
     // of the live rows [0, perm_count) holds original row row_orig[k], and row_int is the inverse;
     // steps_since_exchange counts the training steps since the last call that exchanged rows with the
-    // caller (which restores the original order: sxh_detail::canonicalize).
+    // caller and restored the original order (sxh_detail::canonicalize; a download does neither).
     int row_order = SXH_ROW_ORDER_SPATIAL_AUTO;
     bool permuted = false;
     int perm_count = 0;

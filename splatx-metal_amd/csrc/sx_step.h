@@ -172,7 +172,12 @@ int step_ssim_bwd_blocks(int H, int W);
 void step_set_word(uint32_t* word, uint32_t value, hipStream_t s);
 // rb's words to the host without a loss (the loss word is 0): the forward-only step
 void step_readback(const StepReadback& rb, hipStream_t s);
-void aos_to_soa(const float* aos, float* soa, int rows, int dim, int stride, hipStream_t s);
-void soa_to_aos(const float* soa, float* aos, int rows, int dim, int stride, hipStream_t s);
+// Rows of one parameter group (dim columns at stride `stride`) to and from row-major arrays (k_perm.hip).
+// soa_to_rows: row k < n goes to place dst_row[k] (k < n_perm; dst_row null or k >= n_perm: place k), places
+// at or past n_out (default n) left out. rows_to_soa: row k < n comes from place src_row[k] (null: k).
+void soa_to_rows(const float* soa, float* aos, int n, int dim, int stride, hipStream_t s,
+                 const int32_t* dst_row = nullptr, int n_perm = 0, int n_out = -1);
+void rows_to_soa(const float* aos, float* soa, int n, int dim, int stride, hipStream_t s,
+                 const int32_t* src_row = nullptr);
 
 } // namespace sxk
