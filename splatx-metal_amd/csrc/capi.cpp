@@ -63,6 +63,7 @@ int32_t sxh_backend_create(int32_t device_ordinal, sxh_backend** out) {
         try {
             SXH_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
             SXH_HIP(hipHostMalloc(reinterpret_cast<void**>(&b->pinned_word), sizeof(uint32_t), hipHostMallocDefault));
+            b->xfer = std::make_unique<HostXfer>(device_ordinal);
             noalloc_init(device_ordinal);  // the allocation-free entry points' scratch on this device
         } catch (...) {
             sxh_backend_destroy(b);
@@ -74,6 +75,9 @@ int32_t sxh_backend_create(int32_t device_ordinal, sxh_backend** out) {
 
 void sxh_backend_destroy(sxh_backend* b) {
     if (!b) return;
+    if (b->stream) (void)hipStreamSynchronize(b->stream);
+    b->xfer.reset();
+    b->cache.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->pinned_word) (void)hipHostFree(b->pinned_word);
     delete b;
@@ -105,18 +109,18 @@ int32_t sxh_fused_adam(sxh_backend* b, const sxh_adam_inputs* in) {
         if (in->n_elems == 0) return;
         SXH_HIP(hipSetDevice(b->device));
         const size_t n = static_cast<size_t>(in->n_elems);
-        auto p = upload(in->param, n, b->stream);
-        auto g = upload(in->grad, n, b->stream);
-        auto m = upload(in->exp_avg, n, b->stream);
-        auto v = upload(in->exp_avg_sq, n, b->stream);
+        auto p = upload(in->param, n, b);
+        auto g = upload(in->grad, n, b);
+        auto m = upload(in->exp_avg, n, b);
+        auto v = upload(in->exp_avg_sq, n, b);
         DevBuf<uint8_t> valid;
-        if (in->valid) valid = upload(in->valid, static_cast<size_t>(in->n_gauss), b->stream);
+        if (in->valid) valid = upload(in->valid, static_cast<size_t>(in->n_gauss), b);
         sxk::adam(p.p, g.p, m.p, v.p, valid.p, in->n_elems, in->n_elems / in->n_gauss, in->lr, in->b1, in->b2,
                   in->eps, b->stream);
         SXH_HIP(hipGetLastError());
-        download(in->param, p, n, b->stream);
-        download(in->exp_avg, m, n, b->stream);
-        download(in->exp_avg_sq, v, n, b->stream);
+        download(in->param, p, n, b);
+        download(in->exp_avg, m, n, b);
+        download(in->exp_avg_sq, v, n, b);
         sync(b);
     });
 }
@@ -135,29 +139,29 @@ int32_t sxh_projection_fused_fwd(sxh_backend* b, const sxh_projection_inputs* in
         if (CN == 0) return;
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto means = upload(in->means, N * 3, s);
+        auto means = upload(in->means, N * 3, b);
         DevBuf<float> covars, quats, scales, opac;
-        if (in->covars) covars = upload(in->covars, N * 6, s);
+        if (in->covars) covars = upload(in->covars, N * 6, b);
         else {
-            quats = upload(in->quats, N * 4, s);
-            scales = upload(in->scales, N * 3, s);
+            quats = upload(in->quats, N * 4, b);
+            scales = upload(in->scales, N * 3, b);
         }
-        if (in->opacities) opac = upload(in->opacities, N, s);
-        auto vm = upload(in->viewmats, C * 16, s);
-        auto K = upload(in->Ks, C * 9, s);
-        auto radii = zeros<int32_t>(CN * 2, s);
-        auto m2 = zeros<float>(CN * 2, s);
-        auto dep = zeros<float>(CN, s);
-        auto con = zeros<float>(CN * 3, s);
-        auto comp = zeros<float>(in->calc_compensations ? CN : 0, s);
+        if (in->opacities) opac = upload(in->opacities, N, b);
+        auto vm = upload(in->viewmats, C * 16, b);
+        auto K = upload(in->Ks, C * 9, b);
+        auto radii = zeros<int32_t>(CN * 2, b);
+        auto m2 = zeros<float>(CN * 2, b);
+        auto dep = zeros<float>(CN, b);
+        auto con = zeros<float>(CN * 3, b);
+        auto comp = zeros<float>(in->calc_compensations ? CN : 0, b);
         sxk::projection_fwd(proj_args(*in, means.p, covars.p, quats.p, scales.p, opac.p, vm.p, K.p), radii.p, m2.p,
                             dep.p, con.p, comp.p, s);
         SXH_HIP(hipGetLastError());
-        download(out->radii, radii, CN * 2, s);
-        download(out->means2d, m2, CN * 2, s);
-        download(out->depths, dep, CN, s);
-        download(out->conics, con, CN * 3, s);
-        if (in->calc_compensations) download(out->compensations, comp, CN, s);
+        download(out->radii, radii, CN * 2, b);
+        download(out->means2d, m2, CN * 2, b);
+        download(out->depths, dep, CN, b);
+        download(out->conics, con, CN * 3, b);
+        if (in->calc_compensations) download(out->compensations, comp, CN, b);
         sync(b);
     });
 }
@@ -182,40 +186,40 @@ int32_t sxh_projection_fused_bwd(sxh_backend* b, const sxh_projection_inputs* in
         need(b, "projection_fused_bwd", "backend");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto means = upload(in->means, N * 3, s);
+        auto means = upload(in->means, N * 3, b);
         DevBuf<float> covars, quats, scales, comps, vcomps;
-        if (cov) covars = upload(in->covars, N * 6, s);
+        if (cov) covars = upload(in->covars, N * 6, b);
         else {
-            quats = upload(in->quats, N * 4, s);
-            scales = upload(in->scales, N * 3, s);
+            quats = upload(in->quats, N * 4, b);
+            scales = upload(in->scales, N * 3, b);
         }
-        auto vm = upload(in->viewmats, C * 16, s);
-        auto K = upload(in->Ks, C * 9, s);
-        auto radii = upload(g->radii, CN * 2, s);
-        auto con = upload(g->conics, CN * 3, s);
+        auto vm = upload(in->viewmats, C * 16, b);
+        auto K = upload(in->Ks, C * 9, b);
+        auto radii = upload(g->radii, CN * 2, b);
+        auto con = upload(g->conics, CN * 3, b);
         if (g->v_compensations) {
-            comps = upload(g->compensations, CN, s);
-            vcomps = upload(g->v_compensations, CN, s);
+            comps = upload(g->compensations, CN, b);
+            vcomps = upload(g->v_compensations, CN, b);
         }
-        auto vm2 = upload(g->v_means2d, CN * 2, s);
-        auto vdep = upload(g->v_depths, CN, s);
-        auto vcon = upload(g->v_conics, CN * 3, s);
-        auto v_means = zeros<float>(N * 3, s);
-        auto v_covars = zeros<float>(cov ? N * 6 : 0, s);
-        auto v_quats = zeros<float>(cov ? 0 : N * 4, s);
-        auto v_scales = zeros<float>(cov ? 0 : N * 3, s);
-        auto v_view = zeros<float>(g->viewmats_grad ? C * 16 : 0, s);
+        auto vm2 = upload(g->v_means2d, CN * 2, b);
+        auto vdep = upload(g->v_depths, CN, b);
+        auto vcon = upload(g->v_conics, CN * 3, b);
+        auto v_means = zeros<float>(N * 3, b);
+        auto v_covars = zeros<float>(cov ? N * 6 : 0, b);
+        auto v_quats = zeros<float>(cov ? 0 : N * 4, b);
+        auto v_scales = zeros<float>(cov ? 0 : N * 3, b);
+        auto v_view = zeros<float>(g->viewmats_grad ? C * 16 : 0, b);
         sxk::ProjBwdArgs ga{radii.p, con.p, comps.p, vm2.p, vdep.p, vcon.p, vcomps.p, g->viewmats_grad ? 1 : 0};
         sxk::projection_bwd(proj_args(*in, means.p, covars.p, quats.p, scales.p, nullptr, vm.p, K.p), ga,
                             v_means.p, v_covars.p, v_quats.p, v_scales.p, v_view.p, s);
         SXH_HIP(hipGetLastError());
-        download(out->v_means, v_means, N * 3, s);
-        if (cov) download(out->v_covars, v_covars, N * 6, s);
+        download(out->v_means, v_means, N * 3, b);
+        if (cov) download(out->v_covars, v_covars, N * 6, b);
         else {
-            download(out->v_quats, v_quats, N * 4, s);
-            download(out->v_scales, v_scales, N * 3, s);
+            download(out->v_quats, v_quats, N * 4, b);
+            download(out->v_scales, v_scales, N * 3, b);
         }
-        if (g->viewmats_grad) download(out->v_viewmats, v_view, C * 16, s);
+        if (g->viewmats_grad) download(out->v_viewmats, v_view, C * 16, b);
         sync(b);
     });
 }
@@ -231,16 +235,16 @@ int32_t sxh_sh_fwd(sxh_backend* b, const sxh_sh_inputs* in, float* colors) {
         need(colors, "sh_fwd", "colors");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto dirs = upload(in->dirs, BN * 3, s);
-        auto co = upload(in->coeffs, static_cast<size_t>(in->N * in->K) * in->D, s);
+        auto dirs = upload(in->dirs, BN * 3, b);
+        auto co = upload(in->coeffs, static_cast<size_t>(in->N * in->K) * in->D, b);
         DevBuf<uint8_t> masks;
-        if (in->masks) masks = upload(in->masks, BN, s);
+        if (in->masks) masks = upload(in->masks, BN, b);
         // masked elements are left unwritten: stage the caller's buffer so untouched slots survive
-        auto out = upload(colors, BN * in->D, s);
+        auto out = upload(colors, BN * in->D, b);
         sxk::sh_fwd(dirs.p, co.p, masks.p, in->degrees_to_use, static_cast<int>(in->B), static_cast<int>(in->N),
                     static_cast<int>(in->K), static_cast<int>(in->D), out.p, s);
         SXH_HIP(hipGetLastError());
-        download(colors, out, BN * in->D, s);
+        download(colors, out, BN * in->D, b);
         sync(b);
     });
 }
@@ -261,19 +265,19 @@ int32_t sxh_sh_bwd(sxh_backend* b, const sxh_sh_inputs* in, const float* v_color
         need(v_colors, "sh_bwd", "v_colors");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto dirs = upload(in->dirs, BN * 3, s);
-        auto co = upload(in->coeffs, NKD, s);
+        auto dirs = upload(in->dirs, BN * 3, b);
+        auto co = upload(in->coeffs, NKD, b);
         DevBuf<uint8_t> masks;
-        if (in->masks) masks = upload(in->masks, BN, s);
-        auto vc = upload(v_colors, BN * in->D, s);
-        auto vco = zeros<float>(NKD, s);
-        auto vd = zeros<float>(in->compute_v_dirs ? BN * 3 : 0, s);
+        if (in->masks) masks = upload(in->masks, BN, b);
+        auto vc = upload(v_colors, BN * in->D, b);
+        auto vco = zeros<float>(NKD, b);
+        auto vd = zeros<float>(in->compute_v_dirs ? BN * 3 : 0, b);
         sxk::sh_bwd(dirs.p, co.p, masks.p, in->degrees_to_use, static_cast<int>(in->B), static_cast<int>(in->N),
                     static_cast<int>(in->K), static_cast<int>(in->D), vc.p, vco.p,
                     in->compute_v_dirs ? vd.p : nullptr, s);
         SXH_HIP(hipGetLastError());
-        download(v_coeffs, vco, NKD, s);
-        if (in->compute_v_dirs) download(v_dirs, vd, BN * 3, s);
+        download(v_coeffs, vco, NKD, b);
+        if (in->compute_v_dirs) download(v_dirs, vd, BN * 3, b);
         sync(b);
     });
 }
@@ -294,17 +298,17 @@ int32_t sxh_isect_tiles(sxh_backend* b, const sxh_isect_inputs* in, sxh_isect_ou
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
         const size_t n = static_cast<size_t>(n_el);
-        auto m2 = upload(in->means2d, n * 2, s);
-        auto radii = upload(in->radii, n * 2, s);
-        auto dep = upload(in->depths, n, s);
+        auto m2 = upload(in->means2d, n * 2, b);
+        auto radii = upload(in->radii, n * 2, b);
+        auto dep = upload(in->depths, n, b);
         DevBuf<float> con, op;
         if (in->conics) {
-            con = upload(in->conics, n * 3, s);
-            op = upload(in->opacities, n, s);
+            con = upload(in->conics, n * 3, b);
+            op = upload(in->opacities, n, b);
         }
-        DevBuf<int32_t> tiles(n);
-        DevBuf<int64_t> cum(n);
-        DevBuf<uint8_t> scratch(sxk::scan_scratch_bytes(n_el));
+        DevBuf<int32_t> tiles(n, &b->cache);
+        DevBuf<int64_t> cum(n, &b->cache);
+        DevBuf<uint8_t> scratch(sxk::scan_scratch_bytes(n_el), &b->cache);
         sxk::IsectArgs a{m2.p, radii.p, dep.p, con.p, op.p, static_cast<int>(in->I), static_cast<int>(in->N),
                          static_cast<int>(in->tile_size), static_cast<int>(in->tile_width),
                          static_cast<int>(in->tile_height), out->tile_n_bits};
@@ -312,7 +316,7 @@ int32_t sxh_isect_tiles(sxh_backend* b, const sxh_isect_inputs* in, sxh_isect_ou
         sxk::isect_count(a, tiles.p, s);
         sxk::scan_i32_i64(tiles.p, cum.p, n_el, scratch.p, s);
         SXH_HIP(hipGetLastError());
-        download(out->tiles_per_gauss, tiles, n, s);
+        download(out->tiles_per_gauss, tiles, n, b);
         int64_t total = 0;
         SXH_HIP(hipMemcpyAsync(&total, cum.p + (n - 1), sizeof(int64_t), hipMemcpyDeviceToHost, s));
         sync(b);
@@ -326,12 +330,12 @@ int32_t sxh_isect_tiles(sxh_backend* b, const sxh_isect_inputs* in, sxh_isect_ou
                                 std::to_string(total));
         need(out->isect_ids, "isect_tiles", "isect_ids");
         need(out->flatten_ids, "isect_tiles", "flatten_ids");
-        DevBuf<uint64_t> keys(static_cast<size_t>(total));
-        DevBuf<int32_t> vals(static_cast<size_t>(total));
+        DevBuf<uint64_t> keys(static_cast<size_t>(total), &b->cache);
+        DevBuf<int32_t> vals(static_cast<size_t>(total), &b->cache);
         sxk::isect_emit(a, cum.p, keys.p, vals.p, s);
         SXH_HIP(hipGetLastError());
-        download(out->isect_ids, keys, static_cast<size_t>(total), s);
-        download(out->flatten_ids, vals, static_cast<size_t>(total), s);
+        download(out->isect_ids, keys, static_cast<size_t>(total), b);
+        download(out->flatten_ids, vals, static_cast<size_t>(total), b);
         sync(b);
     });
 }
@@ -345,12 +349,12 @@ int32_t sxh_prefix_scan_i64(sxh_backend* b, const int32_t* in, int64_t n, int64_
         need(out, "prefix_scan_i64", "out");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto d_in = upload(in, static_cast<size_t>(n), s);
-        DevBuf<int64_t> d_out(static_cast<size_t>(n));
-        DevBuf<uint8_t> scratch(sxk::scan_scratch_bytes(n));
+        auto d_in = upload(in, static_cast<size_t>(n), b);
+        DevBuf<int64_t> d_out(static_cast<size_t>(n), &b->cache);
+        DevBuf<uint8_t> scratch(sxk::scan_scratch_bytes(n), &b->cache);
         sxk::scan_i32_i64(d_in.p, d_out.p, n, scratch.p, s);
         SXH_HIP(hipGetLastError());
-        download(out, d_out, static_cast<size_t>(n), s);
+        download(out, d_out, static_cast<size_t>(n), b);
         sync(b);
     });
 }
@@ -366,19 +370,19 @@ int32_t sxh_sort_isect(sxh_backend* b, const sxh_sort_inputs* in, uint64_t* keys
         need(values_sorted, "sort_isect", "values_sorted");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto ka = upload(in->keys, n, s);
-        auto va = upload(in->values, n, s);
-        DevBuf<uint64_t> kb(n);
-        DevBuf<int32_t> vb(n);
-        DevBuf<uint8_t> scratch(sxk::sort_scratch_bytes(in->n));
+        auto ka = upload(in->keys, n, b);
+        auto va = upload(in->values, n, b);
+        DevBuf<uint64_t> kb(n, &b->cache);
+        DevBuf<int32_t> vb(n, &b->cache);
+        DevBuf<uint8_t> scratch(sxk::sort_scratch_bytes(in->n), &b->cache);
         const int which = sxk::radix_sort(ka.p, va.p, kb.p, vb.p, in->n, in->key_n_bits, scratch.p, s);
         uint32_t sort_err = 0;
         SXH_HIP(hipMemcpyAsync(&sort_err, sxk::sort_error_flag(scratch.p), 4, hipMemcpyDeviceToHost, s));
         SXH_HIP(hipStreamSynchronize(s));
         if (sort_err) throw std::runtime_error("sort_isect: radix sort look-back did not complete");
         SXH_HIP(hipGetLastError());
-        download(keys_sorted, which ? kb : ka, n, s);
-        download(values_sorted, which ? vb : va, n, s);
+        download(keys_sorted, which ? kb : ka, n, b);
+        download(values_sorted, which ? vb : va, n, b);
         sync(b);
     });
 }
@@ -406,12 +410,12 @@ int32_t sxh_isect_offset_encode(sxh_backend* b, const sxh_offset_inputs* in, int
         }
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto keys = upload(in->isect_ids, static_cast<size_t>(in->n_isects), s);
-        auto off = zeros<int32_t>(total, s);
+        auto keys = upload(in->isect_ids, static_cast<size_t>(in->n_isects), b);
+        auto off = zeros<int32_t>(total, b);
         sxk::offset_encode(keys.p, in->n_isects, static_cast<int>(in->I), static_cast<int>(n_tiles),
                            sx::bits_for_count(n_tiles), off.p, s);
         SXH_HIP(hipGetLastError());
-        download(offsets, off, total, s);
+        download(offsets, off, total, b);
         sync(b);
     });
 }
@@ -425,7 +429,8 @@ struct RasterStage {
     DevBuf<uint8_t> masks;
     sxk::RasterArgs args{};
 };
-void stage_raster(const sxh_raster_inputs& in, hipStream_t s, RasterStage& st) {
+void stage_raster(const sxh_raster_inputs& in, sxh_backend* b, RasterStage& st) {
+    hipStream_t s = b->stream;
     const size_t n = static_cast<size_t>(in.I * in.N);
     const size_t n_tiles = static_cast<size_t>(in.tile_width) * in.tile_height;
     // Index inputs are caller data: keep every device gather in bounds.
@@ -435,16 +440,16 @@ void stage_raster(const sxh_raster_inputs& in, hipStream_t s, RasterStage& st) {
     for (int64_t k = 0; k < in.n_isects; k++)
         if (in.flatten_ids[k] < 0 || static_cast<size_t>(in.flatten_ids[k]) >= n)
             invalid("rasterize", "flatten_ids[" + std::to_string(k) + "] outside [0, I*N)");
-    auto m2 = upload(in.means2d, n * 2, s);
-    auto cn = upload(in.conics, n * 3, s);
-    auto col = upload(in.colors, n * 3, s);
-    auto op = upload(in.opacities, n, s);
-    st.splats.alloc(std::max<size_t>(n, 1) * 3);
+    auto m2 = upload(in.means2d, n * 2, b);
+    auto cn = upload(in.conics, n * 3, b);
+    auto col = upload(in.colors, n * 3, b);
+    auto op = upload(in.opacities, n, b);
+    st.splats = DevBuf<float4>(std::max<size_t>(n, 1) * 3, &b->cache);
     sxk::pack_splats(m2.p, cn.p, col.p, op.p, static_cast<int>(n), st.splats.p, s);
-    st.offsets = upload(in.isect_offsets, static_cast<size_t>(in.I) * n_tiles, s);
-    if (in.n_isects > 0) st.flat = upload(in.flatten_ids, static_cast<size_t>(in.n_isects), s);
-    if (in.backgrounds) st.bg = upload(in.backgrounds, static_cast<size_t>(in.I) * 3, s);
-    if (in.masks) st.masks = upload(in.masks, static_cast<size_t>(in.I) * n_tiles, s);
+    st.offsets = upload(in.isect_offsets, static_cast<size_t>(in.I) * n_tiles, b);
+    if (in.n_isects > 0) st.flat = upload(in.flatten_ids, static_cast<size_t>(in.n_isects), b);
+    if (in.backgrounds) st.bg = upload(in.backgrounds, static_cast<size_t>(in.I) * 3, b);
+    if (in.masks) st.masks = upload(in.masks, static_cast<size_t>(in.I) * n_tiles, b);
     st.args.splats = st.splats.p;
     st.args.offsets = st.offsets.p;
     st.args.flatten_ids = st.flat.p;
@@ -472,14 +477,14 @@ int32_t sxh_rasterize_fwd(sxh_backend* b, const sxh_raster_inputs* in, sxh_raste
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
         RasterStage st;
-        stage_raster(*in, s, st);
-        DevBuf<float> rgb(P * 3), alpha(P);
-        DevBuf<int32_t> last(P);
+        stage_raster(*in, b, st);
+        DevBuf<float> rgb(P * 3, &b->cache), alpha(P, &b->cache);
+        DevBuf<int32_t> last(P, &b->cache);
         sxk::raster_fwd(st.args, rgb.p, alpha.p, last.p, s);  // always runs: background of empty tiles
         SXH_HIP(hipGetLastError());
-        download(out->render_colors, rgb, P * 3, s);
-        download(out->render_alphas, alpha, P, s);
-        download(out->last_ids, last, P, s);
+        download(out->render_colors, rgb, P * 3, b);
+        download(out->render_alphas, alpha, P, b);
+        download(out->last_ids, last, P, b);
         sync(b);
     });
 }
@@ -500,28 +505,28 @@ int32_t sxh_rasterize_bwd(sxh_backend* b, const sxh_raster_inputs* in, const sxh
         need(b, "rasterize_bwd", "backend");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto vm2 = zeros<float>(n * 2, s);
-        auto vcn = zeros<float>(n * 3, s);
-        auto vcol = zeros<float>(n * 3, s);
-        auto vop = zeros<float>(n, s);
-        auto vabs = zeros<float>(g->absgrad ? n * 2 : 0, s);
+        auto vm2 = zeros<float>(n * 2, b);
+        auto vcn = zeros<float>(n * 3, b);
+        auto vcol = zeros<float>(n * 3, b);
+        auto vop = zeros<float>(n, b);
+        auto vabs = zeros<float>(g->absgrad ? n * 2 : 0, b);
         if (in->n_isects > 0 && P > 0) {
             RasterStage st;
-            stage_raster(*in, s, st);
-            auto ra = upload(g->render_alphas, P, s);
-            auto li = upload(g->last_ids, P, s);
-            auto vrc = upload(g->v_render_colors, P * 3, s);
-            auto vra = upload(g->v_render_alphas, P, s);
+            stage_raster(*in, b, st);
+            auto ra = upload(g->render_alphas, P, b);
+            auto li = upload(g->last_ids, P, b);
+            auto vrc = upload(g->v_render_colors, P * 3, b);
+            auto vra = upload(g->v_render_alphas, P, b);
             sxk::RasterBwdGrads gg{vm2.p, vcn.p, vcol.p, vop.p, g->absgrad ? vabs.p : nullptr, nullptr};
             sxk::raster_bwd(st.args, ra.p, li.p, vrc.p, vra.p, gg, s);
             SXH_HIP(hipGetLastError());
             sync(b);
         }
-        download(out->v_means2d, vm2, n * 2, s);
-        download(out->v_conics, vcn, n * 3, s);
-        download(out->v_colors, vcol, n * 3, s);
-        download(out->v_opacities, vop, n, s);
-        if (g->absgrad) download(out->v_means2d_abs, vabs, n * 2, s);
+        download(out->v_means2d, vm2, n * 2, b);
+        download(out->v_conics, vcn, n * 3, b);
+        download(out->v_colors, vcol, n * 3, b);
+        download(out->v_opacities, vop, n, b);
+        if (g->absgrad) download(out->v_means2d_abs, vabs, n * 2, b);
         sync(b);
     });
 }
@@ -535,10 +540,10 @@ int32_t sxh_rng_normal_f32(sxh_backend* b, const sxh_rng_inputs* in, float* out)
         if (in->count == 0) return;
         need(out, "rng_normal_f32", "out");
         SXH_HIP(hipSetDevice(b->device));
-        DevBuf<float> d(static_cast<size_t>(in->count));
+        DevBuf<float> d(static_cast<size_t>(in->count), &b->cache);
         sxk::rng_normal_f32(in->seed, in->offset, in->count, d.p, b->stream);
         SXH_HIP(hipGetLastError());
-        download(out, d, static_cast<size_t>(in->count), b->stream);
+        download(out, d, static_cast<size_t>(in->count), b);
         sync(b);
     });
 }
@@ -551,10 +556,10 @@ int32_t sxh_rng_philox_u32(sxh_backend* b, const sxh_rng_inputs* in, uint32_t* o
         if (in->count == 0) return;
         need(out, "rng_philox_u32", "out");
         SXH_HIP(hipSetDevice(b->device));
-        DevBuf<uint32_t> d(static_cast<size_t>(in->count));
+        DevBuf<uint32_t> d(static_cast<size_t>(in->count), &b->cache);
         sxk::rng_philox_u32(in->seed, in->offset, in->count, d.p, b->stream);
         SXH_HIP(hipGetLastError());
-        download(out, d, static_cast<size_t>(in->count), b->stream);
+        download(out, d, static_cast<size_t>(in->count), b);
         sync(b);
     });
 }
@@ -574,15 +579,15 @@ int32_t sxh_mcmc_relocation(sxh_backend* b, const sxh_relocation_inputs* in, flo
                 invalid("mcmc_relocation", "ratios[" + std::to_string(i) + "] out of [1, n_max] (host clamp contract)");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto op = upload(in->opacities, N, s);
-        auto sc = upload(in->scales, N * 3, s);
-        auto ra = upload(in->ratios, N, s);
-        auto bi = upload(in->binoms, static_cast<size_t>(in->n_max) * in->n_max, s);
-        DevBuf<float> no(N), ns(N * 3);
+        auto op = upload(in->opacities, N, b);
+        auto sc = upload(in->scales, N * 3, b);
+        auto ra = upload(in->ratios, N, b);
+        auto bi = upload(in->binoms, static_cast<size_t>(in->n_max) * in->n_max, b);
+        DevBuf<float> no(N, &b->cache), ns(N * 3, &b->cache);
         sxk::mcmc_relocation(op.p, sc.p, ra.p, bi.p, static_cast<int>(N), in->n_max, in->min_opacity, no.p, ns.p, s);
         SXH_HIP(hipGetLastError());
-        download(new_op, no, N, s);
-        download(new_sc, ns, N * 3, s);
+        download(new_op, no, N, b);
+        download(new_sc, ns, N * 3, b);
         sync(b);
     });
 }
@@ -596,14 +601,14 @@ int32_t sxh_mcmc_perturb_positions(sxh_backend* b, const sxh_perturb_inputs* in)
         const size_t N = static_cast<size_t>(in->N);
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto pos = upload(in->positions, N * 3, s);
-        auto q = upload(in->quats, N * 4, s);
-        auto sl = upload(in->scales_log, N * 3, s);
-        auto lg = upload(in->opacities_logit, N, s);
-        auto nz = upload(in->noise, N * 3, s);
+        auto pos = upload(in->positions, N * 3, b);
+        auto q = upload(in->quats, N * 4, b);
+        auto sl = upload(in->scales_log, N * 3, b);
+        auto lg = upload(in->opacities_logit, N, b);
+        auto nz = upload(in->noise, N * 3, b);
         sxk::mcmc_perturb(pos.p, q.p, sl.p, lg.p, nz.p, static_cast<int>(N), in->noise_scale, in->t, in->k, s);
         SXH_HIP(hipGetLastError());
-        download(in->positions, pos, N * 3, s);
+        download(in->positions, pos, N * 3, b);
         sync(b);
     });
 }
@@ -623,16 +628,17 @@ int32_t sxh_ssim_fwd(sxh_backend* b, const sxh_ssim_inputs* in, sxh_ssim_outputs
         need(b, "ssim_fwd", "backend");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto a = upload(in->img1, n, s);
-        auto g = upload(in->img2, n, s);
-        DevBuf<float> map(M), mu(in->need_coeffs ? M : 0), sg(in->need_coeffs ? M : 0), cr(in->need_coeffs ? M : 0);
+        auto a = upload(in->img1, n, b);
+        auto g = upload(in->img2, n, b);
+        const size_t Mc = in->need_coeffs ? M : 0;
+        DevBuf<float> map(M, &b->cache), mu(Mc, &b->cache), sg(Mc, &b->cache), cr(Mc, &b->cache);
         sxk::ssim_fwd(a.p, g.p, I, H, W, C, in->need_coeffs ? 1 : 0, map.p, mu.p, sg.p, cr.p, nullptr, s);
         SXH_HIP(hipGetLastError());
-        download(out->ssim_map, map, M, s);
+        download(out->ssim_map, map, M, b);
         if (in->need_coeffs) {
-            download(out->coeff_mu, mu, M, s);
-            download(out->coeff_sigma, sg, M, s);
-            download(out->coeff_cross, cr, M, s);
+            download(out->coeff_mu, mu, M, b);
+            download(out->coeff_sigma, sg, M, b);
+            download(out->coeff_cross, cr, M, b);
         }
         sync(b);
         double sum = 0.0;  // ssim_reduce_mean_f64 (CpuKernels.h:198-202): ascending-index f64 sum
@@ -655,16 +661,16 @@ int32_t sxh_ssim_bwd(sxh_backend* b, const sxh_ssim_inputs* in, const sxh_ssim_g
         need(b, "ssim_bwd", "backend");
         SXH_HIP(hipSetDevice(b->device));
         hipStream_t s = b->stream;
-        auto a = upload(in->img1, n, s);
-        auto g = upload(in->img2, n, s);
-        auto mu = upload(gin->coeff_mu, M, s);
-        auto sg = upload(gin->coeff_sigma, M, s);
-        auto cr = upload(gin->coeff_cross, M, s);
-        DevBuf<float> v(n);
+        auto a = upload(in->img1, n, b);
+        auto g = upload(in->img2, n, b);
+        auto mu = upload(gin->coeff_mu, M, b);
+        auto sg = upload(gin->coeff_sigma, M, b);
+        auto cr = upload(gin->coeff_cross, M, b);
+        DevBuf<float> v(n, &b->cache);
         const float G = static_cast<float>(-static_cast<double>(gin->v_loss) / static_cast<double>(M));
         sxk::ssim_bwd(a.p, g.p, mu.p, sg.p, cr.p, I, H, W, C, G, v.p, s);
         SXH_HIP(hipGetLastError());
-        download(v_img1, v, n, s);
+        download(v_img1, v, n, b);
         sync(b);
     });
 }

@@ -82,7 +82,10 @@ int32_t sxh_exec_create(sxh_backend* b, const sxh_exec_desc* desc, sxh_executor*
             e->blk_base.alloc(2 * static_cast<size_t>(sxk::step_preprocess_blocks(desc->arena_rows)));
             e->emit_list.alloc(R);
             e->loss_dev.alloc(1);
-            e->staging.alloc(R * 45);
+            // one group of rows at a time; a small arena's parameters and moments together, so that they travel as
+            // one block (65,536 rows at SH3: 46 MB)
+            constexpr size_t kOneBlockRows = 1 << 16;
+            e->staging.alloc(R * (R <= kOneBlockRows ? 3 * (14 + 45) : 45));
             e->ensure_isect(1 << 16);
             const char* dbg = std::getenv("SXH_DEBUG_FORCE_SORT_ERROR");
             e->debug_sort_error = dbg && dbg[0] == '1';
@@ -111,6 +114,10 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
     if (!s) invalid("TrainStepExecutor", "null sync");
     if (s->rows < 0 || s->rows > e->rows) invalid("TrainStepExecutor", "sync rows out of [0, arena_rows]");
     const int rows = static_cast<int>(s->rows);
+    if (rows > 0)
+        for (int g = 0; g < 6; g++)
+            if (e->dims[g] > 0 && (!s->params[g] || !s->exp_avg[g] || !s->exp_avg_sq[g]))
+                invalid("TrainStepExecutor", "null parameter/moment pointer for group " + std::to_string(g));
     if (up && !(e->permuted && rows >= e->perm_count)) {
         sxh_detail::canonicalize(e);  // rows in the caller's order, the pending update applied
     } else {
@@ -127,24 +134,30 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
     const int n_pack = e->permuted ? std::max(rows, e->perm_count) : rows;
     const int32_t* const place = e->permuted ? e->row_orig.p : nullptr;
     hipStream_t st = e->b->stream;
+    std::vector<XferItem> items;
+    int64_t floats = 0;
+    for (int g = 0; g < 6; g++) floats += static_cast<int64_t>(rows) * e->dims[g] * 3;
+    const bool one_block = static_cast<size_t>(floats) <= e->staging.n;
+    float* at = e->staging.p;
     for (int g = 0; g < 6; g++) {
         const int dim = e->dims[g];
         if (dim == 0) continue;
-        float* host[3] = {s->params[g], s->exp_avg[g], s->exp_avg_sq[g]};
-        DevBuf<float>* dev[3] = {&e->p[g], &e->m[g], &e->v[g]};
+        float* const host[3] = {s->params[g], s->exp_avg[g], s->exp_avg_sq[g]};
+        float* const dev[3] = {e->p[g].p, e->m[g].p, e->v[g].p};
         for (int k = 0; k < 3; k++) {
-            if (!host[k]) invalid("TrainStepExecutor", "null parameter/moment pointer for group " + std::to_string(g));
-            const size_t n = static_cast<size_t>(rows) * dim;
-            if (up) {
-                SXH_HIP(hipMemcpyAsync(e->staging.p, host[k], n * 4, hipMemcpyHostToDevice, st));
-                sxk::rows_to_soa(e->staging.p, dev[k]->p, rows, dim, e->rows, st);
-            } else {
-                sxk::soa_to_rows(dev[k]->p, e->staging.p, n_pack, dim, e->rows, st, place, e->perm_count, rows);
-                SXH_HIP(hipMemcpyAsync(host[k], e->staging.p, n * 4, hipMemcpyDeviceToHost, st));
-            }
-            SXH_HIP(hipStreamSynchronize(st));  // staging is reused
+            // (side by side where the staging buffer holds all; else one after another in it, in stream order)
+            XferItem it{host[k], at, static_cast<size_t>(rows) * dim * 4, {}};
+            float* const col = dev[k];
+            if (up) it.stage = [=] { sxk::rows_to_soa(at, col, rows, dim, e->rows, st); };
+            else it.stage = [=] { sxk::soa_to_rows(col, at, n_pack, dim, e->rows, st, place, e->perm_count, rows); };
+            items.push_back(std::move(it));
+            if (one_block) at += static_cast<size_t>(rows) * dim;
         }
     }
+    if (up) e->b->xfer->to_device(items, st);
+    else e->b->xfer->to_host(items, st);
+    SXH_HIP(hipGetLastError());
+    SXH_HIP(hipStreamSynchronize(st));
 }
 
 int32_t sxh_exec_upload(sxh_executor* e, const sxh_param_sync* s) {
@@ -170,7 +183,7 @@ int32_t sxh_exec_set_gt_cache(sxh_executor* e, const float* images, int32_t n, i
         SXH_HIP(hipSetDevice(e->b->device));
         const size_t per = static_cast<size_t>(width) * height * 3;
         e->gt_cache.alloc(per * n);
-        SXH_HIP(hipMemcpyAsync(e->gt_cache.p, images, per * n * 4, hipMemcpyHostToDevice, e->b->stream));
+        e->b->xfer->to_device({{const_cast<float*>(images), e->gt_cache.p, per * n * 4, {}}}, e->b->stream);
         SXH_HIP(hipStreamSynchronize(e->b->stream));
         e->gt_n = n;
         e->gt_w = width;
@@ -426,7 +439,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         if (use_gt_cache) {
             gt = e->gt_cache.p + static_cast<size_t>(in->gt_index) * n_px;
         } else {
-            SXH_HIP(hipMemcpyAsync(e->gt_stage.p, in->gt_rgb, n_px * 4, hipMemcpyHostToDevice, s));
+            e->b->xfer->to_device({{const_cast<float*>(in->gt_rgb), e->gt_stage.p, n_px * 4, {}}}, s);
             gt = e->gt_stage.p;
         }
     };
@@ -629,12 +642,10 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
             SXH_HIP(hipGraphDestroy(g));
         }
     };
-    // the render's copies, after segment B
+    // the render's device copy, after segment B
     auto launch_tail = [&]() {
         if (render_to_dev)
             SXH_HIP(hipMemcpyAsync(render_to_dev, e->render.p, n_px * 4, hipMemcpyDeviceToDevice, s));
-        if (out->render_colors)
-            SXH_HIP(hipMemcpyAsync(out->render_colors, e->render.p, n_px * 4, hipMemcpyDeviceToHost, s));
         SXH_HIP(hipGetLastError());
     };
 
@@ -698,6 +709,8 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
     const auto t0 = std::chrono::steady_clock::now();
     if (!e->prof && !e->prof_stats && !render_to_dev && !out->render_colors)
         wait_count_word(hc + 5, seq, s, what);
+    else if (out->render_colors)
+        e->b->xfer->to_host({{out->render_colors, e->render.p, n_px * 4, {}}}, s);
     else
         SXH_HIP(hipStreamSynchronize(s));
     e->sync_ms[1] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -525,12 +525,17 @@ int32_t sxh_render_session_open(sxh_backend* b, const sxh_render_session_args* a
             if (sxh_exec_create(b, &d, &sess->e) != SXH_OK) throw std::runtime_error(sxh_last_error());
             sxh_executor* e = sess->e;
             hipStream_t s = b->stream;
+            std::vector<XferItem> items;
             for (int g = 0; g < 6; g++) {  // parameters only; the moments stay zero
                 if (e->dims[g] == 0) continue;
-                SXH_HIP(hipMemcpyAsync(e->staging.p, c.g[g].data(), c.g[g].size() * 4, hipMemcpyHostToDevice, s));
-                sxk::rows_to_soa(e->staging.p, e->p[g].p, static_cast<int>(c.count), e->dims[g], e->rows, s);
-                SXH_HIP(hipStreamSynchronize(s));
+                items.push_back({c.g[g].data(), e->staging.p, c.g[g].size() * 4, [=, &c] {
+                                     sxk::rows_to_soa(e->staging.p, e->p[g].p, static_cast<int>(c.count), e->dims[g],
+                                                      e->rows, s);
+                                 }});
             }
+            b->xfer->to_device(items, s);
+            SXH_HIP(hipGetLastError());
+            SXH_HIP(hipStreamSynchronize(s));
         } catch (...) {
             if (sess->e) sxh_exec_destroy(sess->e);
             delete sess;
@@ -567,8 +572,7 @@ int32_t sxh_render_session_frame(sxh_render_session* sess, const float* viewmat,
         sess->rgba.ensure(n_px);
         sxk::rgba8(e->render.p, static_cast<int64_t>(n_px), sess->rgba.p, e->b->stream);
         SXH_HIP(hipGetLastError());
-        SXH_HIP(hipMemcpyAsync(out_rgba, sess->rgba.p, n_px * 4, hipMemcpyDeviceToHost, e->b->stream));
-        SXH_HIP(hipStreamSynchronize(e->b->stream));
+        e->b->xfer->to_host({{out_rgba, sess->rgba.p, n_px * 4, {}}}, e->b->stream);
     });
 }
 

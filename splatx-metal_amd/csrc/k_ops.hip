@@ -547,4 +547,31 @@ void mcmc_perturb(float* positions, const float* quats, const float* slog, const
                        noise_scale, t, k);
 }
 
+namespace {
+// 16 B per thread and round where both sides allow it, 4 B otherwise, single bytes past the last whole word
+__global__ void __launch_bounds__(256) k_copy_bytes(char* __restrict__ dst, const char* __restrict__ src, size_t bytes,
+                                                    int word) {
+    const size_t t = blockIdx.x * (size_t)256 + threadIdx.x, step = gridDim.x * (size_t)256;
+    const size_t whole = bytes / word;
+    if (word == 16)
+        for (size_t k = t; k < whole; k += step) reinterpret_cast<uint4*>(dst)[k] = reinterpret_cast<const uint4*>(src)[k];
+    else if (word == 4)
+        for (size_t k = t; k < whole; k += step)
+            reinterpret_cast<uint32_t*>(dst)[k] = reinterpret_cast<const uint32_t*>(src)[k];
+    else
+        for (size_t k = t; k < whole; k += step) dst[k] = src[k];
+    const size_t k = whole * word + t;
+    if (k < bytes) dst[k] = src[k];
+}
+} // namespace
+
+void copy_bytes(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes == 0) return;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src);
+    const int word = a % 16 == 0 ? 16 : a % 4 == 0 ? 4 : 1;
+    const size_t n = std::max<size_t>(1, bytes / word);
+    hipLaunchKernelGGL(k_copy_bytes, dim3(static_cast<unsigned>(std::min<size_t>(1024, (n + 255) / 256))), dim3(256), 0, s,
+                       static_cast<char*>(dst), static_cast<const char*>(src), bytes, word);
+}
+
 } // namespace sxk

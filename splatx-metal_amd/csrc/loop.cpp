@@ -201,13 +201,14 @@ int64_t filtered_rows(sxh_executor* e, int64_t count, std::vector<float> (&host)
     int64_t kept = 0;
     SXH_HIP(hipMemcpyAsync(&kept, e->cum.p + (N - 1), 8, hipMemcpyDeviceToHost, s));
     SXH_HIP(hipStreamSynchronize(s));
+    std::vector<XferItem> items;
     for (int g = 0; g < 6; g++) {
         host[g].assign(static_cast<size_t>(kept) * e->dims[g], 0.0f);
         if (!kept || !e->dims[g]) continue;
-        sxk::gather_rows(A.p[g], e->rows, e->dims[g], list.p, kept, e->staging.p, s);
-        SXH_HIP(hipMemcpyAsync(host[g].data(), e->staging.p, host[g].size() * 4, hipMemcpyDeviceToHost, s));
+        items.push_back({host[g].data(), e->staging.p, host[g].size() * 4,
+                         [=, &list] { sxk::gather_rows(A.p[g], e->rows, e->dims[g], list.p, kept, e->staging.p, s); }});
     }
-    SXH_HIP(hipStreamSynchronize(s));
+    e->b->xfer->to_host(items, s);
     return kept;
 }
 

@@ -136,16 +136,16 @@ int32_t sxh_running_sum_f64(sxh_backend* b, const float* w, int64_t n, double* o
         if (n == 0) return;
         if (!w || !out) invalid("running_sum_f64", "null w/out");
         SXH_HIP(hipSetDevice(b->device));
-        auto dw = upload(w, static_cast<size_t>(n), b->stream);
-        DevBuf<double> cdf(static_cast<size_t>(n)), total(1);
-        DevBuf<uint32_t> err(1);
-        DevBuf<uint8_t> scratch(sxk::mc_cdf_scratch_bytes(n));
+        auto dw = upload(w, static_cast<size_t>(n), b);
+        DevBuf<double> cdf(static_cast<size_t>(n), &b->cache), total(1, &b->cache);
+        DevBuf<uint32_t> err(1, &b->cache);
+        DevBuf<uint8_t> scratch(sxk::mc_cdf_scratch_bytes(n), &b->cache);
         sxk::fill_u32(err.p, 0u, 1, b->stream);
         sxk::mc_cdf(dw.p, nullptr, n, cdf.p, total.p, err.p, scratch.p, b->stream);
         SXH_HIP(hipGetLastError());
         uint32_t herr = 0;
         SXH_HIP(hipMemcpyAsync(&herr, err.p, 4, hipMemcpyDeviceToHost, b->stream));
-        download(out, cdf, static_cast<size_t>(n), b->stream);
+        download(out, cdf, static_cast<size_t>(n), b);
         SXH_HIP(hipStreamSynchronize(b->stream));
         if (herr & sxk::kMcErrWeights) invalid("running_sum_f64", "weights must be >= 0 and finite");
     });
@@ -159,7 +159,8 @@ int32_t sxh_mt64_draw(sxh_backend* b, sxh_mt64_state* st, int64_t n, uint64_t* o
         if (n == 0) return;
         if (!out) invalid("mt64_draw", "null out");
         SXH_HIP(hipSetDevice(b->device));
-        DevBuf<uint64_t> state(kMtWords + 1), raw(static_cast<size_t>(n)), tempered(static_cast<size_t>(n));
+        DevBuf<uint64_t> state(kMtWords + 1, &b->cache), raw(static_cast<size_t>(n), &b->cache),
+            tempered(static_cast<size_t>(n), &b->cache);
         uint64_t host_state[kMtWords + 1];
         std::memcpy(host_state, st->x, sizeof(st->x));
         host_state[kMtWords] = st->p;
@@ -167,7 +168,7 @@ int32_t sxh_mt64_draw(sxh_backend* b, sxh_mt64_state* st, int64_t n, uint64_t* o
         sxk::mc_mt_gen(state.p, n, raw.p, b->stream);
         sxk::mc_temper(raw.p, n, tempered.p, b->stream);
         SXH_HIP(hipGetLastError());
-        download(out, tempered, static_cast<size_t>(n), b->stream);
+        download(out, tempered, static_cast<size_t>(n), b);
         SXH_HIP(hipMemcpyAsync(host_state, state.p, sizeof(host_state), hipMemcpyDeviceToHost, b->stream));
         SXH_HIP(hipStreamSynchronize(b->stream));
         std::memcpy(st->x, host_state, sizeof(st->x));

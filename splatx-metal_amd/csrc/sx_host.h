@@ -10,12 +10,16 @@
 
 #include <cstdint>
 #include <cstring>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
 
 #include "splatx_hip.h"
 #include "sx_common.h"
+#include "sx_xfer.h"
 
 namespace sxh {
 
@@ -58,53 +62,103 @@ int32_t guarded(F&& f) {
     }
 }
 
-// Owning device allocation.
+// Device memory that the per-op entry points used before, kept for their next calls: at most kMost bytes, given
+// back with the backend. The entry points run on the backend's one stream, so a block is used again in stream
+// order. (hipMalloc and hipFree take 10-100 us each, and an entry point has up to twelve buffers.)
+class DevCache {
+  public:
+    DevCache() = default;
+    DevCache(const DevCache&) = delete;
+    DevCache& operator=(const DevCache&) = delete;
+    ~DevCache() { release(); }
+    void* get(size_t bytes, size_t* got) {
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            const auto it = free_.lower_bound(bytes);
+            if (it != free_.end() && it->first <= 2 * bytes + 4096) {
+                void* p = it->second;
+                *got = it->first;
+                held_ -= it->first;
+                free_.erase(it);
+                return p;
+            }
+        }
+        // (rounded up, so that calls of about the same size share blocks)
+        *got = (bytes + bytes / 8 + 4095) & ~size_t{4095};
+        void* p = nullptr;
+        if (hipMalloc(&p, *got) == hipSuccess) return p;
+        (void)hipGetLastError();
+        release();
+        SXH_HIP(hipMalloc(&p, *got));
+        return p;
+    }
+    void put(void* p, size_t bytes) {
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            if (held_ + bytes <= kMost) {
+                free_.emplace(bytes, p);
+                held_ += bytes;
+                return;
+            }
+        }
+        (void)hipFree(p);
+    }
+    void release() {
+        std::lock_guard<std::mutex> g(mu_);
+        for (const auto& f : free_) (void)hipFree(f.second);
+        free_.clear();
+        held_ = 0;
+    }
+
+  private:
+    static constexpr size_t kMost = size_t{256} << 20;
+    std::mutex mu_;
+    std::multimap<size_t, void*> free_;
+    size_t held_ = 0;
+};
+
+// Owning device allocation; with a cache, its memory comes from there and goes back there.
 template <class T>
 struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
+    DevCache* home = nullptr;
+    size_t home_bytes = 0;
     DevBuf() = default;
-    explicit DevBuf(size_t count) { alloc(count); }
+    explicit DevBuf(size_t count, DevCache* cache = nullptr) : home(cache) { alloc(count); }
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), home(o.home), home_bytes(o.home_bytes) { o.p = nullptr; o.n = 0; }
     DevBuf& operator=(DevBuf&& o) noexcept {
-        if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+        if (this != &o) {
+            release();
+            p = o.p; n = o.n; home = o.home; home_bytes = o.home_bytes;
+            o.p = nullptr; o.n = 0;
+        }
         return *this;
     }
     ~DevBuf() { release(); }
     void alloc(size_t count) {
         release();
+        if (!count) return;
+        const size_t bytes = std::max<size_t>(count * sizeof(T), 16);
+        if (home) p = static_cast<T*>(home->get(bytes, &home_bytes));
+        else SXH_HIP(hipMalloc(reinterpret_cast<void**>(&p), bytes));
         n = count;
-        if (count) SXH_HIP(hipMalloc(reinterpret_cast<void**>(&p), std::max<size_t>(count * sizeof(T), 16)));
     }
     void ensure(size_t count) {
         if (count > n) alloc(count);
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (home) home->put(p, home_bytes);
+            else (void)hipFree(p);
+        }
         p = nullptr;
         n = 0;
     }
     size_t bytes() const { return n * sizeof(T); }
 };
-
-template <class T>
-DevBuf<T> upload(const T* host, size_t count, hipStream_t s) {
-    DevBuf<T> d(count);
-    if (count && host) SXH_HIP(hipMemcpyAsync(d.p, host, count * sizeof(T), hipMemcpyHostToDevice, s));
-    return d;
-}
-template <class T>
-DevBuf<T> zeros(size_t count, hipStream_t s) {
-    DevBuf<T> d(count);
-    if (count) SXH_HIP(hipMemsetAsync(d.p, 0, count * sizeof(T), s));
-    return d;
-}
-template <class T>
-void download(T* host, const DevBuf<T>& d, size_t count, hipStream_t s) {
-    if (count && host) SXH_HIP(hipMemcpyAsync(host, d.p, count * sizeof(T), hipMemcpyDeviceToHost, s));
-}
 
 // ---- validators (Validate.h) -----------------------------------------------------------------
 inline void validate_adam(const sxh_adam_inputs& in, const char* what) {
@@ -240,7 +294,29 @@ struct sxh_backend {
     hipStream_t stream = nullptr;
     std::string name;
     uint32_t* pinned_word = nullptr;  // a pinned host word for status readbacks of the allocation-free calls
+    std::unique_ptr<sxh::HostXfer> xfer;  // copies of the callers' arrays
+    sxh::DevCache cache;                  // the per-op entry points' device buffers
 };
+
+namespace sxh {
+// The per-op entry points' buffers: a device copy of a host array, a zeroed array, an array back to the host.
+template <class T>
+DevBuf<T> upload(const T* host, size_t count, sxh_backend* b) {
+    DevBuf<T> d(count, &b->cache);
+    if (count && host) b->xfer->to_device({{const_cast<T*>(host), d.p, count * sizeof(T), {}}}, b->stream);
+    return d;
+}
+template <class T>
+DevBuf<T> zeros(size_t count, sxh_backend* b) {
+    DevBuf<T> d(count, &b->cache);
+    if (count) SXH_HIP(hipMemsetAsync(d.p, 0, count * sizeof(T), b->stream));
+    return d;
+}
+template <class T>
+void download(T* host, const DevBuf<T>& d, size_t count, sxh_backend* b) {
+    if (count && host) b->xfer->to_host({{host, d.p, count * sizeof(T), {}}}, b->stream);
+}
+}  // namespace sxh
 
 namespace sxh {
 // Resolves the allocation-free entry points' scratch array on `device` (the current device).

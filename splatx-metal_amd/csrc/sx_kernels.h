@@ -253,4 +253,7 @@ void mcmc_relocation(const float* opac, const float* scales, const int32_t* rati
 void mcmc_perturb(float* positions, const float* quats, const float* scales_log, const float* logits,
                   const float* noise, int N, float noise_scale, float t, float k, hipStream_t s);
 
+// A copy by a kernel on the stream, between device memory and mapped host memory of any alignment
+void copy_bytes(void* dst, const void* src, size_t bytes, hipStream_t s);
+
 } // namespace sxk
