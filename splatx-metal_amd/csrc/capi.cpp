@@ -62,7 +62,6 @@ int32_t sxh_backend_create(int32_t device_ordinal, sxh_backend** out) {
         b->name = std::string("hip-gfx950:") + prop.gcnArchName;
         try {
             SXH_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-            SXH_HIP(hipHostMalloc(reinterpret_cast<void**>(&b->pinned_word), sizeof(uint32_t), hipHostMallocDefault));
             b->xfer = std::make_unique<HostXfer>(device_ordinal);
             noalloc_init(device_ordinal);  // the allocation-free entry points' scratch on this device
         } catch (...) {
@@ -79,7 +78,6 @@ void sxh_backend_destroy(sxh_backend* b) {
     b->xfer.reset();
     b->cache.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
-    if (b->pinned_word) (void)hipHostFree(b->pinned_word);
     delete b;
 }
 
@@ -376,10 +374,6 @@ int32_t sxh_sort_isect(sxh_backend* b, const sxh_sort_inputs* in, uint64_t* keys
         DevBuf<int32_t> vb(n, &b->cache);
         DevBuf<uint8_t> scratch(sxk::sort_scratch_bytes(in->n), &b->cache);
         const int which = sxk::radix_sort(ka.p, va.p, kb.p, vb.p, in->n, in->key_n_bits, scratch.p, s);
-        uint32_t sort_err = 0;
-        SXH_HIP(hipMemcpyAsync(&sort_err, sxk::sort_error_flag(scratch.p), 4, hipMemcpyDeviceToHost, s));
-        SXH_HIP(hipStreamSynchronize(s));
-        if (sort_err) throw std::runtime_error("sort_isect: radix sort look-back did not complete");
         SXH_HIP(hipGetLastError());
         download(keys_sorted, which ? kb : ka, n, b);
         download(values_sorted, which ? vb : va, n, b);

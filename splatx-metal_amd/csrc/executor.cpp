@@ -306,7 +306,7 @@ static void spatial_order(sxh_executor* e, int count) {
     const sxk::Arena A = e->arena();
     sxk::arena_morton_keys(A, count, e->perm_scratch.p, e->dkey_a.p, e->order_a.p, s);
     const int w = sxk::radix_sort(e->dkey_a.p, e->order_a.p, e->dkey_b.p, e->order_b.p, count, 30, e->sort_scratch.p, s,
-                                  true, nullptr, true);
+                                  true, nullptr);
     if (w < 0) throw std::runtime_error("TrainStepExecutor: spatial order sort failed");
     const int32_t* src = w ? e->order_b.p : e->order_a.p;
     sxk::arena_permute_rows(A, e->dims, count, src, e->staging.p, s);
@@ -467,9 +467,8 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         const int32_t* order = e->emit_list.p;
         if (!index_first) {
             sxk::step_depth_keys(c, e->splats.p, e->emit_list.p, n_emit, e->dkey_a.p, e->order_a.p, s);
-            // (the step's sorts never wait on another workgroup: they cannot give up halfway through a step)
             const int wd = sxk::radix_sort(e->dkey_a.p, e->order_a.p, e->dkey_b.p, e->order_b.p, c.count, 32,
-                                           e->sort_scratch.p, s, true, n_emit_i, true);
+                                           e->sort_scratch.p, s, true, n_emit_i);
             if (wd < 0) throw std::runtime_error(std::string(what) + ": arena too large for a device-count depth sort");
             order = wd ? e->order_b.p : e->order_a.p;
             e->mark("depth_sort");
@@ -484,6 +483,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         uint32_t* const edepth_b =
             index_first ? reinterpret_cast<uint32_t*>(e->keys_a.p) + e->isect_cap : nullptr;
         int which = 0;
+        sxk::DigitStarts starts{e->offsets.p, n_tiles, false};  // (up to 256 tiles the sort leaves the offsets)
         if (c.tile_n_bits <= 16) {
             uint16_t* ka = reinterpret_cast<uint16_t*>(e->keys_a.p);
             uint16_t* kb = reinterpret_cast<uint16_t*>(e->keys_b.p);
@@ -495,9 +495,9 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                                       edepth);
             e->mark("emit");
             which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
-                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, true);
+                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &starts);
             e->mark("sort");
-            sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
+            if (!starts.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
         } else {
             uint32_t* ka = reinterpret_cast<uint32_t*>(e->keys_a.p);
             uint32_t* kb = reinterpret_cast<uint32_t*>(e->keys_b.p);
@@ -509,9 +509,9 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                                       edepth);
             e->mark("emit");
             which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
-                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, true);
+                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &starts);
             e->mark("sort");
-            sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
+            if (!starts.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
         }
         if (which < 0) throw std::runtime_error(std::string(what) + ": intersection capacity too large for a device count");
         if (e->debug_sort_error) sxk::step_set_word(sxk::sort_error_flag(e->sort_scratch.p), 1u, s);
@@ -728,7 +728,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                                           st[sxk::kStatBwdEntries],     st[sxk::kStatBwdEmptyChunks],
                                           st[sxk::kStatBwdInCutoff],    st[sxk::kStatBwdContrib]};
     }
-    if (sort_err) throw std::runtime_error(std::string(what) + ": radix sort look-back did not complete");
+    if (sort_err) throw std::runtime_error(std::string(what) + ": radix sort did not complete");
     if (e->prof) {
         sxh_exec_timing& t = e->timing;
         t.n = 0;

@@ -2,14 +2,12 @@
 // keys of sort_isect), u32 (depths) or u16 (tile ids).
 //
 // Contract: KernelBackend.h:130-148 / sort_isect (ascending unsigned key, stable, only bits
-// [0, key_bits) significant). Design: digits of at most 8 bits, the key bits spread evenly over the
-// fewest passes, so a 45-bit isect key needs 6 passes (the reference's 4-bit digits need 12) and a
-// 13-bit tile id two passes (6 then 7 bits; 7 then 6 in onesweep). Below 16 tiles of 4096 keys the passes run onesweep (see
-// k_os_pass): the digit histograms of all passes come from one read of the keys, and each pass is one
-// launch whose tiles chain their digit prefixes by look-back. From 16 tiles (and below 2^30 keys) on
-// each pass counts its tiles' digits, scans the count matrix and scatters with the same pass kernel,
-// without the chain (see k_rs_count). The fallback at 2^30 keys and above is three launches per pass
-// with no inter-workgroup waiting:
+// [0, key_bits) significant). Design: digits of at most 8 bits (u64 keys 9), the key bits spread evenly over the
+// fewest passes, so a 45-bit isect key needs 5 passes (the reference's 4-bit digits need 12) and a
+// 13-bit tile id two (6 then 7 bits). A pass counts each tile's digits and places its keys with the counts of the
+// tiles before it. Up to kRowKeys keys that is two launches (k_row_count, k_pass); above, and below 2^30 keys, the
+// count matrix is scanned between them (k_rs_count, k_rs_reduce, k_rs_down, k_pass); no workgroup waits on
+// another. The fallback at 2^30 keys and above is three launches per pass:
 //   1. per-tile digit histogram (LDS counters)        -> hist[digit][tile], plus the digit totals
 //   2. one workgroup per digit scans its row of hist   -> global start of (digit, tile)
 //   3. stable scatter: each 64-lane wave ranks the keys of its quarter of the tile per digit with 8
@@ -33,7 +31,6 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kRounds = 16;
 constexpr int kTile = kThreads * kRounds;  // 4096 keys per workgroup
 constexpr int kBins = 256;
-constexpr int kMaxPassesOs = 8;
 constexpr int kXcds = 8;  // XCDs of an MI355X (workgroups are dealt to them round-robin)
 
 // Pass p of a sort on bits [0, key_bits) with digits of `dbits` bits covers bits [p dbits, p dbits +
@@ -93,6 +90,7 @@ __global__ void __launch_bounds__(kThreads) k_zero_totals(uint32_t* __restrict__
     if (err && threadIdx.x == 0) *err = 0u;
 }
 
+template <int W = kWaves>
 __device__ inline uint32_t block_excl_scan_u32(uint32_t v, uint32_t* s_wave, uint32_t* total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t x = v;
@@ -105,7 +103,7 @@ __device__ inline uint32_t block_excl_scan_u32(uint32_t v, uint32_t* s_wave, uin
     __syncthreads();
     uint32_t pre = 0, tot = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) {
+    for (int w = 0; w < W; w++) {
         if (w < wave) pre += s_wave[w];
         tot += s_wave[w];
     }
@@ -251,158 +249,6 @@ __global__ void __launch_bounds__(kThreads) k_scatter(const K* __restrict__ kin,
     }
 }
 
-// ---- onesweep: one launch per pass (digit histograms of every pass from one read up front) ----
-// Tile t of a pass publishes its digit counts to status[t][d] as soon as it has ranked its keys
-// (flag AGG), then looks back over its predecessors' words, adding counts until it meets an
-// inclusive prefix (flag INC), and publishes its own inclusive prefix. Tiles take their index from
-// an atomic counter in the order they start, so every tile a tile waits on has already started and
-// publishes without waiting itself: the look-back always ends. A bounded spin turns a broken
-// invariant into an error flag instead of a hang.
-constexpr uint32_t kFlagAgg = 1u << 30;
-constexpr uint32_t kFlagInc = 2u << 30;
-constexpr uint32_t kValMask = (1u << 30) - 1u;
-constexpr uint32_t kSpinLimit = 1u << 20;
-constexpr int kLook = 8;  // predecessor words per lane and look-back round trip
-// A pass with 2^w < 256 digit values gives each digit G = min(256 / 2^w, kLookLanes) adjacent lanes
-// for its look-back, so a round trip reads G * kLook predecessors: the chain of inclusive prefixes
-// then advances G times faster, which is what bounds a pass over many tiles.
-constexpr int kLookLanes = 16;
-
-__device__ __forceinline__ uint32_t ld_status(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_status(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Digit histograms of passes [0, passes) -> totals[p][d]; clears the first pass's status words and
-// the per-pass tile counters. Grid-stride over 4096-key chunks. A wave whose 64 digits agree (the
-// tile bits of neighbouring keys) adds once; otherwise each lane adds 1 (spread digits, few
-// collisions): cheaper than match masks here, where no ranks are needed.
-template <class K>
-__global__ void __launch_bounds__(kThreads) k_os_hist(const K* __restrict__ keys, int64_t n, int passes, int dbits, uint32_t key_bits,
-                                                      uint32_t* __restrict__ totals, uint32_t* __restrict__ status0,
-                                                      int64_t status_words, uint32_t* __restrict__ counters,
-                                                      const int64_t* __restrict__ n_dev) {
-    __shared__ uint32_t h[kMaxPassesOs][kBins];
-    if (n_dev) {
-        n = *n_dev;
-        status_words = (n + kTile - 1) / kTile * kBins;
-    }
-    for (int p = 0; p < kMaxPassesOs; p++) h[p][threadIdx.x] = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < status_words; i += (int64_t)gridDim.x * kThreads)
-        status0[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < kMaxPassesOs) counters[threadIdx.x] = 0u;
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int64_t chunks = (n + kTile - 1) / kTile;
-    for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        const int64_t base = c * kTile;
-        K key[kRounds];  // the whole chunk in flight before any counting
-#pragma unroll
-        for (int r = 0; r < kRounds; r++) {
-            const int64_t idx = base + r * kThreads + threadIdx.x;
-            key[r] = idx < n ? keys[idx] : K(0);
-        }
-#pragma unroll
-        for (int r = 0; r < kRounds; r++) {
-            const bool valid = base + r * kThreads + threadIdx.x < n;
-            for (int p = 0; p < passes; p++) {
-                const uint32_t d = static_cast<uint32_t>(key[r] >> (dbits * p)) & digit_mask(p, dbits, key_bits);
-                const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
-                if (__all(valid && d == d0)) {  // one digit for the whole wave: one add
-                    if (lane == 0) atomicAdd(&h[p][d0], 64u);
-                } else if (valid) {
-                    atomicAdd(&h[p][d], 1u);  // spread digits: lanes mostly hit distinct counters
-                }
-            }
-        }
-    }
-    __syncthreads();
-    for (int p = 0; p < passes; p++) {
-        const uint32_t v = h[p][threadIdx.x];
-        if (v) atomicAdd(&totals[p * kBins + threadIdx.x], v);
-    }
-}
-
-// The same digit totals for keys of at most kFullBits significant bits: one LDS counter per key
-// value (2^key_bits of them, dynamic LDS), one add per key, then each pass's digit totals are sums
-// of those counters. With few digit values (a 13-bit tile id sorts as 128 + 64 bins) a wave's 64
-// random keys would collide on the same digit counter and serialize; over 8192 key counters they
-// rarely do, and there is one add per key instead of one per pass.
-constexpr uint32_t kFullBits = 14;
-// blocks of the histogram kernels: each adds its digit counts to the same few totals, and adds to one
-// address serialize, so the grid is kept near the CU count (grid-stride over the chunks)
-constexpr int kHistBlocks = 512;
-template <class K>
-__global__ void __launch_bounds__(kThreads) k_os_hist_full(const K* __restrict__ keys, int64_t n, int passes, int dbits,
-                                                           uint32_t key_bits, uint32_t* __restrict__ totals,
-                                                           uint32_t* __restrict__ status0, int64_t status_words,
-                                                           uint32_t* __restrict__ counters, const int64_t* __restrict__ n_dev) {
-    extern __shared__ uint32_t hf[];
-    __shared__ uint32_t s_dig[kBins];
-    if (n_dev) {
-        n = *n_dev;
-        status_words = (n + kTile - 1) / kTile * kBins;
-    }
-    const uint32_t nb = 1u << key_bits;
-    for (uint32_t i = threadIdx.x; i < nb; i += kThreads) hf[i] = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < status_words; i += (int64_t)gridDim.x * kThreads)
-        status0[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < kMaxPassesOs) counters[threadIdx.x] = 0u;
-    __syncthreads();
-    const uint32_t kmask = nb - 1u;
-    const int64_t chunks = (n + kTile - 1) / kTile;
-    for (int64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
-        const int64_t base = c * kTile;
-        K key[kRounds];
-#pragma unroll
-        for (int r = 0; r < kRounds; r++) {
-            const int64_t idx = base + r * kThreads + threadIdx.x;
-            key[r] = idx < n ? keys[idx] : K(0);
-        }
-#pragma unroll
-        for (int r = 0; r < kRounds; r++)
-            if (base + r * kThreads + threadIdx.x < n) atomicAdd(&hf[static_cast<uint32_t>(key[r]) & kmask], 1u);
-    }
-    __syncthreads();
-    // pass p, digit d (width w at shift s) counts the key values (hi << (s + w)) | (d << s) | lo, i.e.
-    // the j-th of its 2^(key_bits - w) counters is j = hi 2^s + lo; the 256 threads split the digits'
-    // counters evenly and add their partial sums to the totals
-    for (int p = 0; p < passes; p++) {
-        const int s = dbits * p;
-        const uint32_t dm = digit_mask(p, dbits, key_bits);
-        const int w = __popc(dm);
-        const uint32_t per_digit = nb >> w;                        // counters per digit
-        const uint32_t tpd = kThreads >> w;                        // threads per digit (w <= 8)
-        const uint32_t d = threadIdx.x >> (8 - w);                 // this thread's digit
-        const uint32_t span = per_digit / tpd ? per_digit / tpd : 1u;
-        const uint32_t j0 = (threadIdx.x & (tpd - 1)) * span;
-        uint32_t acc = 0;
-        if (j0 < per_digit)
-            for (uint32_t j = j0; j < j0 + span && j < per_digit; j++)
-                acc += hf[((j >> s) << (s + w)) | (d << s) | (j & ((1u << s) - 1u))];
-        // one global add per digit and block: the totals are few addresses that every block adds to,
-        // and adds to one address serialize
-        s_dig[threadIdx.x] = 0;
-        __syncthreads();
-        if (acc) atomicAdd(&s_dig[d], acc);
-        __syncthreads();
-        if (threadIdx.x <= dm && s_dig[threadIdx.x]) atomicAdd(&totals[p * kBins + threadIdx.x], s_dig[threadIdx.x]);
-        __syncthreads();
-    }
-}
-
-// totals[p][d] -> base[p][d] = keys of digits < d (exclusive scan per pass); totals left as is
-__global__ void __launch_bounds__(kThreads) k_os_scan(const uint32_t* __restrict__ totals, int passes,
-                                                      uint32_t* __restrict__ base) {
-    __shared__ uint32_t s_wave[kWaves];
-    for (int p = 0; p < passes; p++) {
-        uint32_t all = 0;
-        base[p * kBins + threadIdx.x] = block_excl_scan_u32(totals[p * kBins + threadIdx.x], s_wave, &all);
-    }
-}
-
 // Lanes of the wave (among `valid_mask`) whose digit, the low NB bits of x, equals this lane's: one
 // ballot per bit, each lane collecting the lanes that differ from it in that bit. Per bit: v_bfe_i32
 // (the bit as 0 or ~0; written as asm, as the compiler otherwise makes a shift pair of it), the ballot's
@@ -432,15 +278,14 @@ __device__ __forceinline__ uint32_t lanes_below_count(uint64_t mask) {
 }
 
 // ---- reduce-then-scan: the pass's prefixes without a chain between tiles ------------------------
-// For sorts of many tiles the onesweep pass is bound by its look-back: a tile waits until its
-// predecessors' inclusive prefixes have been published, which advance at a fixed rate along the chain.
-// Instead each pass counts the digits of every tile (k_rs_count, digit-major: cnt[d][tile]), scans the
+// (One launch per pass whose tiles chain their prefixes by look-back is bound by that chain: config 5's sort
+// took 1.69 ms so and 1.43 with a scan.) Each pass counts the digits of every tile (k_rs_count, digit-major: cnt[d][tile]), scans the
 // whole count matrix once (the exclusive prefix of entry (d, tile) is where the tile's run of digit d
 // starts in the output: all keys of smaller digits, then those of digit d in earlier tiles), and the
 // pass kernel places its keys with these starts. Counts fit u32: a pass sorts fewer than 2^30 keys.
 constexpr int kScanChunk = kThreads * 16;  // elements per workgroup of the count-matrix scan
 
-// Digit counts of tile blockIdx.x -> cnt[d * n_tiles + tile] for d <= mask. Every workgroup of the grid
+// Digit counts of a tile -> cnt[d * n_tiles + tile] for d <= mask. Every workgroup of the grid
 // writes its counts (zeros for a tile past the device count), so the scanned matrix is complete. A
 // thread takes 16 consecutive keys (16-B loads) and adds each run of equal digits once: neighbouring
 // keys often share the high digits (the tiles of one Gaussian along a row), and the lanes of a wave,
@@ -453,7 +298,7 @@ __global__ void __launch_bounds__(kThreads) k_rs_count(const K* __restrict__ key
     static_assert(kRounds * sizeof(K) % 16 == 0, "a thread's keys are whole 16-B vectors");
     __shared__ uint32_t h[kBins];
     if (err && blockIdx.x == 0 && threadIdx.x == 0) *err = 0u;
-    // tiles dealt XCD by XCD, as in k_os_pass (a grid of kXcds * ceil(n_tiles / kXcds)): a digit's counts
+    // tiles dealt XCD by XCD, as in k_pass (a grid of kXcds * ceil(n_tiles / kXcds)): a digit's counts
     // of consecutive tiles are neighbouring words of the matrix, and their partial lines then merge in
     // one L2
     const int per = (n_tiles + kXcds - 1) / kXcds;
@@ -563,22 +408,117 @@ __global__ void __launch_bounds__(kThreads) k_rs_down(uint32_t* __restrict__ v, 
     }
 }
 
-// NB = the digit's width in bits (mask = 2^NB - 1). CHAIN: the onesweep pass (tile index from the
-// counter, prefixes by look-back); otherwise tile = blockIdx.x and the tile's run of digit d starts at
-// starts[d * n_tiles + tile] (the scanned count matrix of the reduce-then-scan path).
+// ---- two launches per pass: the tiles' counts as rows, added up by the pass itself ---------------------
+// Sorts of up to kRowKeys keys are bound by the latency of their launches (2 M u64 keys with a scan of the count
+// matrix between count and pass: those two launches took 7 us of a pass's 28, 70 thousand keys 4.7 of 18.5).
+// Here a tile's digit counts are one row (cnt[tile][T]), the rows of each kGroup tiles are also added up (gsum,
+// integer atomics), and every workgroup of the pass reads the group rows and its own group's rows before it (at
+// most 64 + 31 coalesced rows, in flight during the ranking): their sums are the digit's
+// keys in earlier tiles, and a scan over the digits' totals is where each digit starts. Up to kDirectTiles tiles
+// the tile rows alone. Workgroups of T threads sort digits of up to log2(T) bits: u64 keys take T = 512 (a 45-bit
+// key in five passes instead of six), tile ids and depths 256.
+constexpr int kGroup = 32;
+constexpr int kDirectTiles = 64;
+
+template <class K, int R, int T>
+__global__ void __launch_bounds__(T) k_row_count(const K* __restrict__ keys, int64_t n, int shift, uint32_t mask,
+                                                        uint32_t* __restrict__ cnt, uint32_t* __restrict__ gsum,
+                                                        uint32_t* __restrict__ gsum_next, int n_groups, int n_tiles,
+                                                        const int64_t* __restrict__ n_dev, uint32_t* __restrict__ err) {
+    constexpr int kThreads = T, kBins = T;
+    __shared__ uint32_t h[kBins];
+    if (err && blockIdx.x == 0 && threadIdx.x == 0) *err = 0u;
+    // the next pass's group sums (read by no workgroup of this launch) cleared, a slice per workgroup
+    constexpr int kSlice = kBins / kGroup;
+    if (gsum_next && threadIdx.x < kSlice)
+        for (int k = static_cast<int>(blockIdx.x) * kSlice + threadIdx.x; k < n_groups * kBins; k += gridDim.x * kSlice)
+            gsum_next[k] = 0u;
+    // (tiles dealt XCD by XCD, as in the pass)
+    const int per = (n_tiles + kXcds - 1) / kXcds;
+    const int tile = static_cast<int>(blockIdx.x % kXcds) * per + static_cast<int>(blockIdx.x / kXcds);
+    if (n_dev) n = *n_dev;
+    if (tile >= n_tiles || (int64_t)tile * kThreads * R >= n) return;  // uniform; the pass reads no row past the keys
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t i0 = (int64_t)tile * (kThreads * R) + (int64_t)threadIdx.x * R;
+    K key[R];
+    if (i0 + R <= n) {  // whole vectors: a thread's keys start at a multiple of their size
+        using V = typename std::conditional<R * sizeof(K) % 16 == 0, uint4, uint2>::type;
+        constexpr int kVec = R * sizeof(K) / sizeof(V);
+        static_assert(kVec * sizeof(V) == R * sizeof(K), "a thread's keys are whole vectors");
+        V w[kVec];
+#pragma unroll
+        for (int q = 0; q < kVec; q++) w[q] = reinterpret_cast<const V*>(keys + i0)[q];
+        __builtin_memcpy(key, w, sizeof(key));
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) key[r] = i0 + r < n ? keys[i0 + r] : K(0);
+    }
+    const int valid = static_cast<int>(min<int64_t>(R, max<int64_t>(0, n - i0)));
+    uint32_t run_d = static_cast<uint32_t>(key[0] >> shift) & mask, run_n = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t d = static_cast<uint32_t>(key[r] >> shift) & mask;
+        if (r < valid) {
+            if (d != run_d) {
+                if (run_n) atomicAdd(&h[run_d], run_n);
+                run_d = d;
+                run_n = 0;
+            }
+            run_n++;
+        }
+    }
+    if (run_n) atomicAdd(&h[run_d], run_n);
+    __syncthreads();
+    if (threadIdx.x <= mask) {
+        const uint32_t c = h[threadIdx.x];
+        cnt[(size_t)tile * kBins + threadIdx.x] = c;
+        if (gsum && c) atomicAdd(&gsum[(size_t)(tile / kGroup) * kBins + threadIdx.x], c);
+    }
+}
+
+__global__ void __launch_bounds__(kThreads) k_zero_words(uint32_t* __restrict__ p, int n) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+
+// The sums of rows [0, n) of digit tid (all) and of those below `below` (pre), eight rows in flight.
+template <int T>
+__device__ __forceinline__ void add_rows(const uint32_t* __restrict__ rows, int tid, int n, int below, uint32_t& pre,
+                                         uint32_t& all) {
+    for (int q = 0; q < n; q += 8) {  // uniform
+        uint32_t v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = q + k < n ? rows[(size_t)(q + k) * T + tid] : 0u;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            all += v[k];
+            pre += q + k < below ? v[k] : 0u;
+        }
+    }
+}
+
+// How a pass knows where a tile's run of each digit starts: kMatrix from the scanned count matrix of the
+// reduce-then-scan path (starts[d * n_tiles + tile]), kRows from the tiles' rows of counts (starts = cnt, gsum).
+enum { kMatrix = 0, kRows = 1 };
+constexpr int kLeastBits = 4;  // narrower digits run with four ballots
+
+// One pass: each tile's keys ranked by digit in LDS, reordered there and written out digit by digit.
+// NB = the digit's width in bits (mask = 2^NB - 1; kRows: at most NB bits). R rounds of T keys per tile.
 // X: each key also carries a u32 second value, read from xin at the key's input position and written to
 // xout at its output position (null pointers when X is false). IDX: vin is null, and each key's value is
-// its input position.
-template <class K, int NB, bool CHAIN, bool X, bool IDX>
-__global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin, const int32_t* __restrict__ vin,
-                                                      K* __restrict__ kout, int32_t* __restrict__ vout,
-                                                      int64_t n, int shift, uint32_t mask, const uint32_t* __restrict__ digit_base,
-                                                      uint32_t* __restrict__ status, uint32_t* __restrict__ status_next,
-                                                      uint32_t* __restrict__ counter, uint32_t* __restrict__ err,
-                                                      const int64_t* __restrict__ n_dev,
-                                                      const uint32_t* __restrict__ starts, int n_tiles,
-                                                      const uint32_t* __restrict__ xin, uint32_t* __restrict__ xout) {
-    constexpr int kPerWave = kTile / kWaves;  // 1024
+// its input position. kRows with digit_starts: the pass's first workgroup writes where each digit
+// d < n_starts starts (for keys of one digit, the offset of each key value).
+template <class K, int NB, int MODE, bool X, bool IDX, int R, int T>
+__global__ void __launch_bounds__(T) k_pass(const K* __restrict__ kin, const int32_t* __restrict__ vin,
+                                            K* __restrict__ kout, int32_t* __restrict__ vout, int64_t n, int shift,
+                                            uint32_t mask, const int64_t* __restrict__ n_dev,
+                                            const uint32_t* __restrict__ starts, int n_tiles,
+                                            const uint32_t* __restrict__ xin, uint32_t* __restrict__ xout,
+                                            const uint32_t* __restrict__ gsum, int32_t* __restrict__ digit_starts,
+                                            int n_starts) {
+    constexpr int kThreads = T, kBins = T, kWaves = T / 64, kRounds = R, kTile = T * R;  // this pass's tile
+    constexpr int kPerWave = kTile / kWaves;
     __shared__ K s_k[kTile];
     // IDX (no input values: each key's value is its input position): no value registers, and the LDS
     // reorder moves the keys' 16-bit positions in the tile (83 VGPRs and 22 KB instead of 97 and 30 KB:
@@ -589,16 +529,9 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
     __shared__ uint32_t s_lstart[kBins];
     __shared__ uint32_t s_woff[kWaves][kBins];
     __shared__ uint32_t s_wave[kWaves];
-    __shared__ uint32_t s_cnt[kBins];  // this tile's count of each digit
-    __shared__ uint32_t s_tile;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    if (n_dev) {  // the grid is sized for a capacity: exactly one workgroup per tile of keys takes a tile
-        n = *n_dev;
-        if (CHAIN && static_cast<int64_t>(blockIdx.x) * kTile >= n) return;  // uniform
-    }
-    // CHAIN: one tile, from the counter. Otherwise one tile below the (device) key count, by the
-    // workgroup's index.
+    if (n_dev) n = *n_dev;  // (the grid is sized for a capacity)
     const int64_t n_work = (n + kTile - 1) / kTile;
     // XCD-aware tile order: the GPU deals workgroups to its kXcds XCDs round-robin (workgroup b to XCD
     // b % kXcds, each XCD taking its share in order), so tile (b % kXcds) * per + b / kXcds gives every XCD
@@ -609,15 +542,16 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
     const int64_t per = (n_work + kXcds - 1) / kXcds;
     {
         const int64_t k = blockIdx.x;
-        const int64_t t = CHAIN ? 0 : (k % kXcds) * per + k / kXcds;
-        if (!CHAIN && (k >= per * kXcds || t >= n_work)) return;  // uniform
-        if (CHAIN && tid == 0) s_tile = atomicAdd(counter, 1u);
+        const int64_t t = (k % kXcds) * per + k / kXcds;
+        if (MODE == kRows && digit_starts && n_work == 0 && k == 0)
+            for (int q = tid; q < n_starts; q += kThreads) digit_starts[q] = 0;
+        if (k >= per * kXcds || t >= n_work) return;  // uniform
 #pragma unroll
         for (int w = 0; w < kWaves; w++) s_woff[w][tid] = 0;
         __syncthreads();
-        const uint32_t tile = CHAIN ? s_tile : static_cast<uint32_t>(t);
+        const uint32_t tile = static_cast<uint32_t>(t);
         // the tile's digit starts are requested now, so their latency overlaps the loads and the ranking
-        const uint32_t my_start = (!CHAIN && tid <= mask) ? starts[(size_t)tid * n_tiles + tile] : 0u;
+        uint32_t my_start = (MODE == kMatrix && tid <= mask) ? starts[(size_t)tid * n_tiles + tile] : 0u;
         const int64_t base = (int64_t)tile * kTile;
         const int tile_n = static_cast<int>(min<int64_t>(kTile, n - base));
         K key[kRounds];
@@ -663,6 +597,18 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
                 if (!IDX) val[r] = i < tile_n ? static_cast<int32_t>(base + i) : 0;
             }
         }
+        uint32_t digit_total = 0u;  // kRows: the digit's keys in all tiles (my_start: in the tiles before this one)
+        if (MODE == kRows && tid <= mask) {
+            const int work = static_cast<int>(n_work), first = static_cast<int>(tile) / kGroup * kGroup;
+            if (gsum) {
+                add_rows<T>(gsum, tid, (work + kGroup - 1) / kGroup, first / kGroup, my_start, digit_total);
+                uint32_t sub = 0u, all = 0u;
+                add_rows<T>(starts + (size_t)first * kBins, tid, static_cast<int>(tile) - first, kGroup, sub, all);
+                my_start += sub;
+            } else {
+                add_rows<T>(starts, tid, work, static_cast<int>(tile), my_start, digit_total);
+            }
+        }
         // per-wave digit counts, rounds in order; off[r] = the key's place among the wave's keys of its
         // digit (keys of earlier rounds, then lanes below it with the same digit). All lanes read the
         // digit's running count before one leader lane per digit group advances it.
@@ -671,7 +617,8 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
 #pragma unroll
         for (int r = 0; r < kRounds; r++) {
             const bool valid = wave * kPerWave + r * 64 + lane < tile_n;
-            const uint32_t x = static_cast<uint32_t>(key[r] >> shift);
+            uint32_t x = static_cast<uint32_t>(key[r] >> shift);
+            if (MODE == kRows && NB == kLeastBits) x &= mask;  // (a digit of fewer bits than the ballots)
             const uint32_t d = x & mask;
             const uint64_t match = digit_match_bits<NB>(x, __ballot(valid));
             const uint32_t rank = lanes_below_count(match);
@@ -682,17 +629,20 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
             off[r] = prior + rank;
         }
         __syncthreads();
-        uint32_t tile_count;
         {
-            uint32_t c[kWaves], tot = 0;
+            uint32_t c[kWaves], tot = 0;  // the tile's count of each digit
 #pragma unroll
             for (int w = 0; w < kWaves; w++) {
                 c[w] = s_woff[w][tid];
                 tot += c[w];
             }
-            tile_count = tot;
             uint32_t all = 0;
-            uint32_t run = block_excl_scan_u32(tot, s_wave, &all);
+            if (MODE == kRows) {
+                const uint32_t base_d = block_excl_scan_u32<kWaves>(digit_total, s_wave, &all);
+                my_start += base_d;
+                if (digit_starts && tile == 0u && tid < n_starts) digit_starts[tid] = static_cast<int32_t>(base_d);
+            }
+            uint32_t run = block_excl_scan_u32<kWaves>(tot, s_wave, &all);
             s_lstart[tid] = run;
 #pragma unroll
             for (int w = 0; w < kWaves; w++) {
@@ -700,10 +650,6 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
                 run += c[w];
             }
         }
-        // publish this tile's digit counts now; the look-back for the prefixes of the tiles before it
-        // waits until the tile has been reordered in LDS, which gives them time to finish theirs
-        if (CHAIN) st_status(status + (size_t)tile * kBins + tid, (tile == 0 ? kFlagInc : kFlagAgg) | tile_count);
-        s_cnt[tid] = tile_count;
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < kRounds; r++) {
@@ -716,78 +662,13 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
             }
         }
         __syncthreads();
-        // look back: the G lanes of digit d read kLook predecessors' words each per round trip, lane s
-        // the s-th run of kLook below j, newest first; the group adds counts up to the newest inclusive
-        // prefix among them, or up to the newest word not yet published and retries from there
-        const int bins = static_cast<int>(mask) + 1;
-        const int G = min(kThreads / bins, kLookLanes);  // a power of two dividing 64
-        if (!CHAIN) {
-            if (tid < bins) s_gstart[tid] = my_start - s_lstart[tid];
-        } else if (tile == 0) {
-            s_gstart[tid] = digit_base[tid] - s_lstart[tid];
-        } else if (tid < bins * G) {
-            const int d = tid / G, sub = tid & (G - 1);
-            const int gbase = lane & ~(G - 1);
-            const uint64_t gmask = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;
-            uint32_t excl = 0;
-            int64_t j = (int64_t)tile - 1;
-            uint32_t spins = 0;
-            for (;;) {  // the group's lanes take every branch together
-                const int64_t top = j - (int64_t)sub * kLook;
-                uint32_t w[kLook];
-#pragma unroll
-                for (int q = 0; q < kLook; q++)
-                    w[q] = top - q >= 0 ? ld_status(status + (size_t)(top - q) * kBins + d) : kFlagInc;
-                uint32_t part = 0;
-                int stop = 0, at = kLook;  // stop: 1 = met an inclusive prefix, 2 = met an unpublished word at q = at
-#pragma unroll
-                for (int q = 0; q < kLook; q++) {
-                    if (stop == 0) {
-                        const uint32_t f = w[q] & ~kValMask;
-                        if (f == 0u) {
-                            stop = 2;
-                            at = q;
-                        } else {
-                            part += w[q] & kValMask;
-                            if (f == kFlagInc) stop = 1;
-                        }
-                    }
-                }
-                uint32_t scan = part;  // inclusive over the group's lanes
-                for (int o = 1; o < G; o <<= 1) {
-                    const uint32_t y = __shfl_up(scan, o, 64);
-                    if (sub >= o) scan += y;
-                }
-                const uint64_t stops = __ballot(stop != 0) & gmask;
-                const int first = stops ? static_cast<int>(__builtin_ctzll(stops)) - gbase : G - 1;
-                excl += __shfl(scan, gbase + first, 64);
-                if (!stops) {
-                    j -= (int64_t)G * kLook;
-                    continue;
-                }
-                if (__shfl(stop, gbase + first, 64) == 1) break;
-                const int64_t adv = (int64_t)first * kLook + __shfl(at, gbase + first, 64);
-                j -= adv;
-                if (adv == 0) {
-                    if (++spins > kSpinLimit) {
-                        atomicOr(err, 1u);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-            }
-            if (sub == 0) {
-                st_status(status + (size_t)tile * kBins + d, kFlagInc | (excl + s_cnt[d]));
-                s_gstart[d] = digit_base[d] + excl - s_lstart[d];
-            }
-        }
-        if (CHAIN && status_next) status_next[(size_t)tile * kBins + tid] = 0u;
+        if (tid <= static_cast<int>(mask)) s_gstart[tid] = my_start - s_lstart[tid];
         __syncthreads();
-        const uint32_t n32 = static_cast<uint32_t>(n);  // onesweep runs below 2^30 keys
+        const uint32_t n32 = static_cast<uint32_t>(n);  // (both modes sort fewer than 2^30 keys)
         for (int p = tid; p < tile_n; p += kThreads) {
             const K k = s_k[p];
             const uint32_t g = s_gstart[static_cast<uint32_t>(k >> shift) & mask] + static_cast<uint32_t>(p);
-            if (g < n32) {  // always, unless the look-back gave up (err set): then no write lands out of range
+            if (g < n32) {  // always: no write lands out of range whatever the counts hold
                 kout[g] = k;
                 vout[g] = IDX ? static_cast<int32_t>(base + s_v[p]) : static_cast<int32_t>(s_v[p]);
                 if (X) xout[g] = s_x[p];
@@ -798,36 +679,63 @@ __global__ void __launch_bounds__(kThreads) k_os_pass(const K* __restrict__ kin,
 
 int tiles_for(int64_t n) { return static_cast<int>((n + kTile - 1) / kTile); }
 
-// One onesweep pass over the digit of `mask`'s width at `shift`.
-template <class K, bool CHAIN, bool X = false>
-void launch_os_pass(int tiles, hipStream_t s, const K* kin, const int32_t* vin, K* kout, int32_t* vout, int64_t n,
-                    int shift, uint32_t mask, const uint32_t* digit_base, uint32_t* status, uint32_t* status_next,
-                    uint32_t* counter, uint32_t* err, const int64_t* n_dev, const uint32_t* starts = nullptr,
-                    const uint32_t* xin = nullptr, uint32_t* xout = nullptr) {
-#define SX_OS_PASS(NB)                                                                                          \
-    do {                                                                                                        \
-        if (vin)                                                                                                \
-            hipLaunchKernelGGL((k_os_pass<K, NB, CHAIN, X, false>),                                             \
-                               dim3(CHAIN ? tiles : (tiles + kXcds - 1) / kXcds * kXcds), dim3(kThreads), 0, s, \
-                               kin, vin, kout, vout, n, shift, mask, digit_base, status, status_next, counter,  \
-                               err, n_dev, starts, tiles, xin, xout);                                           \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_os_pass<K, NB, CHAIN, X, true>),                                              \
-                               dim3(CHAIN ? tiles : (tiles + kXcds - 1) / kXcds * kXcds), dim3(kThreads), 0, s, \
-                               kin, vin, kout, vout, n, shift, mask, digit_base, status, status_next, counter,  \
-                               err, n_dev, starts, tiles, xin, xout);                                           \
-    } while (0)
-    switch (__builtin_popcount(mask)) {
-        case 1: SX_OS_PASS(1); break;
-        case 2: SX_OS_PASS(2); break;
-        case 3: SX_OS_PASS(3); break;
-        case 4: SX_OS_PASS(4); break;
-        case 5: SX_OS_PASS(5); break;
-        case 6: SX_OS_PASS(6); break;
-        case 7: SX_OS_PASS(7); break;
-        default: SX_OS_PASS(8); break;
+// The tiles and groups of the two-launch passes over n keys (the capacity, with a device count), for n <= kRowKeys:
+// tiles of 4 T keys up to kSmallKeys, which leave fewer compute units without one and rank four rounds one after
+// another instead of eight, and of 8 T keys above. Measured: a step's tile sort with room for 0.9 M entries, 384 us a
+// step in tiles of 4096, 376 of 1024; with room for 3 M, 47.5 us the sort in tiles of 4096, 44.6 of 2048 (52.6 with
+// the scanned matrix); for 6 M, 85 us in rows of 4096-key tiles, 81 with the matrix, which the line at kRowKeys
+// leaves it to. u64 keys: 1.5 M 115.7 us in tiles of 2048 keys, 2 M 149 and in tiles of 4096 121. groups 0: the tile
+// rows alone.
+constexpr int64_t kRowKeys = int64_t{1} << 22;
+template <class K>
+struct RowPlan {
+    static constexpr int kT = sizeof(K) == 8 ? 512 : 256;
+    static constexpr int kMaxBits = sizeof(K) == 8 ? 9 : 8;
+    static constexpr int64_t kSmallKeys = sizeof(K) == 8 ? 3 << 19 : 1 << 20;
+    int rounds, tiles, groups;
+    bool fits;
+    explicit RowPlan(int64_t n) {
+        fits = n <= kRowKeys;
+        rounds = n <= kSmallKeys ? 4 : 8;
+        const int64_t t = (std::min(n, kRowKeys) + kT * rounds - 1) / (kT * rounds);
+        tiles = static_cast<int>(std::max<int64_t>(t, 1));
+        groups = tiles > kDirectTiles ? (tiles + kGroup - 1) / kGroup : 0;
     }
-#undef SX_OS_PASS
+    size_t words() const { return static_cast<size_t>(tiles + 2 * groups) * kT; }
+    static int passes(uint32_t key_bits) { return static_cast<int>((key_bits + kMaxBits - 1) / kMaxBits); }
+};
+
+
+// One pass over the digit of `mask`'s width at `shift`: the grid covers `tiles` tiles.
+template <class K, int MODE, bool X, int R, int T>
+void launch_pass(int tiles, hipStream_t s, const K* kin, const int32_t* vin, K* kout, int32_t* vout, int64_t n, int shift,
+                 uint32_t mask, const int64_t* n_dev, const uint32_t* starts, const uint32_t* xin, uint32_t* xout,
+                 const uint32_t* gsum = nullptr, int32_t* digit_starts = nullptr, int n_starts = 0) {
+    const dim3 grid((tiles + kXcds - 1) / kXcds * kXcds);
+    auto go = [&](auto nb) {
+        constexpr int NB = decltype(nb)::value;
+        if constexpr ((1 << NB) <= T && (MODE == kMatrix || NB >= kLeastBits)) {
+            // (u64 keys come with their values; the first pass over positions has none)
+            if (vin || sizeof(K) == 8)
+                hipLaunchKernelGGL((k_pass<K, NB, MODE, X, false, R, T>), grid, dim3(T), 0, s, kin, vin, kout, vout, n, shift,
+                                   mask, n_dev, starts, tiles, xin, xout, gsum, digit_starts, n_starts);
+            else if constexpr (sizeof(K) < 8)
+                hipLaunchKernelGGL((k_pass<K, NB, MODE, X, true, R, T>), grid, dim3(T), 0, s, kin, vin, kout, vout, n, shift,
+                                   mask, n_dev, starts, tiles, xin, xout, gsum, digit_starts, n_starts);
+        }
+    };
+    const int bits = __builtin_popcount(mask);
+    switch (MODE == kRows ? std::max(kLeastBits, bits) : bits) {
+        case 1: go(std::integral_constant<int, 1>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 3: go(std::integral_constant<int, 3>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 5: go(std::integral_constant<int, 5>{}); break;
+        case 6: go(std::integral_constant<int, 6>{}); break;
+        case 7: go(std::integral_constant<int, 7>{}); break;
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        default: go(std::integral_constant<int, 9>{}); break;
+    }
 }
 
 // x_dst[i] = x_src[pos[i]] (grid-stride)
@@ -843,16 +751,19 @@ __global__ void __launch_bounds__(kThreads) k_copy_u32(const uint32_t* __restric
 }
 
 constexpr int kMaxPasses = 8;
-// From this many 4096-key tiles on (64 Ki keys) a pass takes its prefixes from a scan of the tiles'
-// digit counts instead of the look-back chain: the counting read costs less than the chain's waits
-// (measured at 143 to 40,557 tiles: config 2's 0.58 M-key tile sort 44.7 -> 39.4 us; the two-launch
-// count scan made the difference at the small sizes).
-constexpr int kRtsMinTiles = 16;
-// scratch layout: a fixed header (digit totals and bases of up to 8 passes, the per-pass tile
-// counters, the error word) and then two tiles x 256 word buffers (the three-launch path's
-// histogram, or the onesweep status words of alternate passes)
-constexpr int kHeaderWords = 2 * kMaxPasses * kBins + 64;
+// scratch layout: a fixed header (digit totals of up to 8 passes, the error word) and then the tiles' counts: rows
+// and their group sums, or a matrix of tiles x 256 words and its scan's chunk sums, or the three-launch path's
+// histogram
+constexpr int kErrWord = kMaxPasses * kBins;
+constexpr int kHeaderWords = kMaxPasses * kBins + 64;
 static_assert(kHeaderWords * sizeof(uint32_t) % 64 == 0, "the count matrix after the header is 64-B aligned");
+
+// The number of passes of a sort of n keys on key_bits bits, of which the two-launch and the count-matrix path make
+// digits of equal widths, give or take one.
+template <class K>
+int sort_passes(int64_t n, uint32_t key_bits) {
+    return RowPlan<K>(n).fits ? RowPlan<K>::passes(key_bits) : static_cast<int>((key_bits + 7) / 8);
+}
 
 // The passes read `src` first and then alternate between the two sides: pass p writes side[p & 1],
 // pass p > 0 reads side[(p - 1) & 1]. src may be side[1] (the sort then works in place over two
@@ -863,91 +774,98 @@ static_assert(kHeaderWords * sizeof(uint32_t) % 64 == 0, "the count matrix after
 // through the passes like the values (pass p writes side_x[p & 1]); the three-launch path, whose
 // scatter does not carry it, gathers it once after the sort through the values, which must then be
 // the input positions (src_v null).
-// no_wait: reduce-then-scan at every size below 2^30 keys (no workgroup ever waits on another, so the
-// sort cannot give up; the onesweep passes below 16 tiles wait on their predecessors with a bounded
-// spin and set the error word if it runs out).
 template <class K>
 int radix_sort_t(const K* src_k, const int32_t* src_v, K* const side_k[2], int32_t* const side_v[2], int64_t n,
                  uint32_t key_bits, void* scratch, bool clear_err, hipStream_t s, const int64_t* n_dev,
-                 const uint32_t* src_x = nullptr, uint32_t* const* side_x = nullptr, bool no_wait = false) {
+                 const uint32_t* src_x = nullptr, uint32_t* const* side_x = nullptr, DigitStarts* ds = nullptr) {
     uint32_t* totals = static_cast<uint32_t*>(scratch);
-    uint32_t* bases = totals + kMaxPasses * kBins;
-    uint32_t* counters = bases + kMaxPasses * kBins;
-    uint32_t* err = counters + kMaxPasses;
+    uint32_t* err = totals + kErrWord;
     key_bits = std::min<uint32_t>(key_bits, 8 * sizeof(K));
-    // fewest 8-bit-or-narrower passes, the bits spread evenly over them (longer runs per digit in each
-    // tile's writes than 8 + 5 for a 13-bit tile id); the onesweep passes take the wider digits first
-    // (7 + 6), the reduce-then-scan passes the narrower ones (6 + 7, below)
-    const int passes = static_cast<int>((key_bits + 7) / 8);
-    const int dbits = passes ? static_cast<int>((key_bits + passes - 1) / passes) : 0;
+    // fewest passes, the bits spread evenly over them (longer runs per digit in each tile's writes than 8 + 5 for
+    // a 13-bit tile id), narrower digits first: the first pass, over keys in the emit's order, has every digit in
+    // each tile and so the shortest runs to write (config 5's 166 M tile ids: 1.026 -> 1.015 ms for the sort)
+    const int passes = sort_passes<K>(n, key_bits);
     if (n <= 0 || passes == 0) {
         if (clear_err) hipLaunchKernelGGL(k_zero_totals, dim3(1), dim3(kThreads), 0, s, totals, 0, err);
         return 0;
     }
     if (n_dev && n >= (int64_t{1} << 30)) return -1;  // the three-launch path sizes its grids by the count
-    const int tiles = std::max(1, tiles_for(n));
-    const int64_t hist_n = (int64_t)tiles * kBins;
+    const int narrow = static_cast<int>(key_bits) / passes, wide_from = passes - static_cast<int>(key_bits) % passes;
+    auto shift_of = [&](int p) { return p * narrow + std::max(0, p - wide_from); };
+    auto mask_of = [&](int p) { return (1u << (narrow + (p >= wide_from ? 1 : 0))) - 1u; };
     uint32_t* hist = totals + kHeaderWords;
-    uint32_t* status_b = hist + hist_n;
     const K* kin = src_k;
     const int32_t* vin = src_v;
-    if (n < (int64_t{1} << 30) && (tiles >= kRtsMinTiles || no_wait)) {  // reduce-then-scan (see k_rs_count)
-        // (the digit totals are not used here; the first count kernel clears the error word)
-        uint32_t* cnt = hist;       // (mask + 1) x tiles counts, then their starts
-        uint32_t* sums = status_b;  // the scan's chunk sums
-        // narrower digits first: the first pass, over keys in the emit's order, has every digit in each
-        // tile and so the shortest runs to write (config 5's 166 M tile ids: 1.026 -> 1.015 ms for the sort)
-        const int narrow = static_cast<int>(key_bits) / passes, wide_from = passes - static_cast<int>(key_bits) % passes;
+    auto x_in = [&](int p) { return !src_x ? nullptr : p == 0 ? src_x : const_cast<const uint32_t*>(side_x[(p - 1) & 1]); };
+    if (const RowPlan<K> rows(n); rows.fits) {  // two launches per pass (see k_row_count)
+        constexpr int T = RowPlan<K>::kT;
+        uint32_t* const cnt = hist;
+        // the passes' group sums in turn: a pass's count clears the next one's
+        uint32_t* const gs[2] = {cnt + (size_t)rows.tiles * T, cnt + (size_t)(rows.tiles + rows.groups) * T};
+        if (rows.groups)
+            hipLaunchKernelGGL(k_zero_words, dim3((rows.groups * T + kThreads - 1) / kThreads), dim3(kThreads), 0, s, gs[0],
+                               rows.groups * T);
+        if (ds) ds->written = passes == 1;
+        auto pass = [&](auto r, auto x, int p) {
+            constexpr int R = decltype(r)::value;
+            constexpr bool X = decltype(x)::value;
+            uint32_t* const g = rows.groups ? gs[p & 1] : nullptr;
+            hipLaunchKernelGGL((k_row_count<K, R, T>), dim3((rows.tiles + kXcds - 1) / kXcds * kXcds), dim3(T), 0, s, kin, n,
+                               shift_of(p), mask_of(p), cnt, g, g && p + 1 < passes ? gs[(p + 1) & 1] : nullptr,
+                               rows.groups, rows.tiles, n_dev, (p == 0 && clear_err) ? err : nullptr);
+            launch_pass<K, kRows, X, R, T>(rows.tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n, shift_of(p), mask_of(p),
+                                           n_dev, cnt, x_in(p), X ? side_x[p & 1] : nullptr, g,
+                                           ds && passes == 1 ? ds->starts : nullptr, ds ? ds->n : 0);
+        };
         for (int p = 0; p < passes; p++) {
-            const int shift = p * narrow + std::max(0, p - wide_from);
-            const uint32_t mask = (1u << (narrow + (p >= wide_from ? 1 : 0))) - 1u;
+            auto with_rounds = [&](auto x) {
+                if (rows.rounds == 4) pass(std::integral_constant<int, 4>{}, x, p);
+                else pass(std::integral_constant<int, 8>{}, x, p);
+            };
+            if constexpr (sizeof(K) < 8) {
+                if (src_x) with_rounds(std::true_type{});
+                else with_rounds(std::false_type{});
+            } else {
+                with_rounds(std::false_type{});
+            }
+            kin = side_k[p & 1];
+            vin = side_v[p & 1];
+        }
+        return passes;
+    }
+    const int tiles = tiles_for(n);
+    if (n < (int64_t{1} << 30)) {  // reduce-then-scan (see k_rs_count)
+        // (the digit totals are not used here; the first count kernel clears the error word)
+        uint32_t* cnt = hist;                                  // (mask + 1) x tiles counts, then their starts
+        uint32_t* sums = hist + (int64_t)tiles * kBins;        // the scan's chunk sums
+        for (int p = 0; p < passes; p++) {
+            const uint32_t mask = mask_of(p);
             const int64_t len = static_cast<int64_t>(mask + 1) * tiles;
             const int chunks = static_cast<int>((len + kScanChunk - 1) / kScanChunk);
             hipLaunchKernelGGL(k_rs_count<K>, dim3((tiles + kXcds - 1) / kXcds * kXcds), dim3(kThreads), 0, s, kin, n,
-                               shift, mask, cnt, tiles, n_dev, (p == 0 && clear_err) ? err : nullptr);
+                               shift_of(p), mask, cnt, tiles, n_dev, (p == 0 && clear_err) ? err : nullptr);
             // (one workgroup scanning a small matrix in one launch measured slower than these)
             hipLaunchKernelGGL(k_rs_reduce, dim3(chunks), dim3(kThreads), 0, s, cnt, len, sums);
             hipLaunchKernelGGL(k_rs_down, dim3(chunks), dim3(kThreads), 0, s, cnt, len, sums);
-            if (src_x)
-                launch_os_pass<K, false, true>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n, shift, mask,
-                                               nullptr, nullptr, nullptr, nullptr, err, n_dev, cnt,
-                                               p == 0 ? src_x : side_x[(p - 1) & 1], side_x[p & 1]);
-            else
-                launch_os_pass<K, false>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n, shift, mask, nullptr,
-                                         nullptr, nullptr, nullptr, err, n_dev, cnt);
+            bool done = false;
+            if constexpr (sizeof(K) < 8) {
+                if (src_x) {
+                    launch_pass<K, kMatrix, true, kRounds, kThreads>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n,
+                                                                     shift_of(p), mask, n_dev, cnt, x_in(p), side_x[p & 1]);
+                    done = true;
+                }
+            }
+            if (!done)
+                launch_pass<K, kMatrix, false, kRounds, kThreads>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n,
+                                                                  shift_of(p), mask, n_dev, cnt, nullptr, nullptr);
             kin = side_k[p & 1];
             vin = side_v[p & 1];
         }
         return passes;
     }
+    const int dbits = static_cast<int>((key_bits + passes - 1) / passes);
     hipLaunchKernelGGL(k_zero_totals, dim3(1), dim3(kThreads), 0, s, totals, passes * kBins,
                        clear_err ? err : nullptr);
-    if (n < (int64_t{1} << 30)) {  // onesweep: counts and prefixes fit the 30-bit status words
-        const int hist_blocks = std::min(tiles, kHistBlocks);
-        if (key_bits <= kFullBits)
-            hipLaunchKernelGGL(k_os_hist_full<K>, dim3(hist_blocks), dim3(kThreads), sizeof(uint32_t) << key_bits, s,
-                               kin, n, passes, dbits, key_bits, totals, hist, hist_n, counters, n_dev);
-        else
-            hipLaunchKernelGGL(k_os_hist<K>, dim3(hist_blocks), dim3(kThreads), 0, s, kin, n, passes, dbits,
-                               key_bits, totals, hist, hist_n, counters, n_dev);
-        hipLaunchKernelGGL(k_os_scan, dim3(1), dim3(kThreads), 0, s, totals, passes, bases);
-        uint32_t* st[2] = {hist, status_b};
-        for (int p = 0; p < passes; p++) {
-            uint32_t* next = p + 1 < passes ? st[(p + 1) & 1] : nullptr;
-            if (src_x)
-                launch_os_pass<K, true, true>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n, dbits * p,
-                                              digit_mask(p, dbits, key_bits), bases + p * kBins, st[p & 1], next,
-                                              counters + p, err, n_dev, nullptr,
-                                              p == 0 ? src_x : side_x[(p - 1) & 1], side_x[p & 1]);
-            else
-                launch_os_pass<K, true>(tiles, s, kin, vin, side_k[p & 1], side_v[p & 1], n, dbits * p,
-                                        digit_mask(p, dbits, key_bits), bases + p * kBins, st[p & 1], next,
-                                        counters + p, err, n_dev);
-            kin = side_k[p & 1];
-            vin = side_v[p & 1];
-        }
-        return passes;
-    }
     for (int p = 0; p < passes; p++) {
         const int shift = dbits * p;
         const uint32_t mask = digit_mask(p, dbits, key_bits);
@@ -979,12 +897,12 @@ int radix_sort_t(const K* src_k, const int32_t* src_v, K* const side_k[2], int32
 template <class K>
 int radix_sort_ab(K* keys_a, int32_t* vals_a, K* keys_b, int32_t* vals_b, int64_t n, uint32_t key_bits,
                   void* scratch, bool clear_err, hipStream_t s, const int64_t* n_dev, bool index_values = false,
-                  uint32_t* x_a = nullptr, uint32_t* x_b = nullptr, bool no_wait = false) {
+                  uint32_t* x_a = nullptr, uint32_t* x_b = nullptr, DigitStarts* ds = nullptr) {
     K* const sk[2] = {keys_b, keys_a};
     int32_t* const sv[2] = {vals_b, vals_a};
     uint32_t* const sx[2] = {x_b, x_a};
     const int passes = radix_sort_t<K>(keys_a, index_values ? nullptr : vals_a, sk, sv, n, key_bits, scratch,
-                                       clear_err, s, n_dev, x_a, x_a ? sx : nullptr, no_wait);
+                                       clear_err, s, n_dev, x_a, x_a ? sx : nullptr, ds);
     return passes < 0 ? -1 : (passes & 1);
 }
 
@@ -994,7 +912,7 @@ int radix_sort_ab(K* keys_a, int32_t* vals_a, K* keys_b, int32_t* vals_b, int64_
 // entry) then gives the order of the reference's (tile | depth) keys: depth, ties by index. One
 // workgroup per tile. A tile of at most 2048 entries is sorted in LDS by 8-bit LSD passes, wave w
 // holding the w-th quarter of the list (in whole 64-key rounds) in registers and ranking with match
-// masks as the onesweep pass does; bytes on which every key of the tile agrees are skipped. A larger
+// masks as the sort's pass does; bytes on which every key of the tile agrees are skipped. A larger
 // tile runs the same passes through global scratch, 2048 keys at a time in list order.
 __device__ __forceinline__ uint32_t wave_and_u32(uint32_t x) {
 #pragma unroll
@@ -1388,13 +1306,16 @@ k_tile_depth_sort(const int32_t* __restrict__ offsets, int n_tiles, int32_t n_is
 } // namespace
 
 size_t sort_scratch_bytes(int64_t n) {
-    const int64_t tiles = std::max<int64_t>(1, tiles_for(n));
-    return sizeof(uint32_t) * static_cast<size_t>(kHeaderWords + 2 * tiles * kBins);
+    const size_t tiles = static_cast<size_t>(std::max(1, tiles_for(n)));
+    size_t words = 2 * tiles * kBins;
+    // (for any key type; a smaller sort in the same scratch may take smaller tiles, so more rows)
+    const int64_t m = std::min(n, kRowKeys);
+    for (const int64_t k : {m, std::min(m, RowPlan<uint16_t>::kSmallKeys)}) words = std::max(words, RowPlan<uint16_t>(k).words());
+    for (const int64_t k : {m, std::min(m, RowPlan<uint64_t>::kSmallKeys)}) words = std::max(words, RowPlan<uint64_t>(k).words());
+    return sizeof(uint32_t) * (kHeaderWords + words);
 }
 
-uint32_t* sort_error_flag(void* scratch) {
-    return static_cast<uint32_t*>(scratch) + 2 * kMaxPasses * kBins + kMaxPasses;
-}
+uint32_t* sort_error_flag(void* scratch) { return static_cast<uint32_t*>(scratch) + kErrWord; }
 
 int radix_sort(uint64_t* keys_a, int32_t* vals_a, uint64_t* keys_b, int32_t* vals_b, int64_t n, uint32_t key_bits,
                void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev) {
@@ -1402,9 +1323,8 @@ int radix_sort(uint64_t* keys_a, int32_t* vals_a, uint64_t* keys_b, int32_t* val
 }
 
 int radix_sort(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n, uint32_t key_bits,
-               void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev, bool no_wait) {
-    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, false, nullptr,
-                         nullptr, no_wait);
+               void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev) {
+    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev);
 }
 
 int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n, uint32_t key_bits,
@@ -1414,16 +1334,14 @@ int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* val
 
 int radix_sort_positions(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev,
-                         uint32_t* x_a, uint32_t* x_b, bool no_wait) {
-    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b,
-                         no_wait);
+                         uint32_t* x_a, uint32_t* x_b, DigitStarts* ds) {
+    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b, ds);
 }
 
 int radix_sort_positions(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev,
-                         uint32_t* x_a, uint32_t* x_b, bool no_wait) {
-    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b,
-                         no_wait);
+                         uint32_t* x_a, uint32_t* x_b, DigitStarts* ds) {
+    return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b, ds);
 }
 
 constexpr int kDepthSortRounds = 8;
@@ -1444,7 +1362,7 @@ void tile_depth_sort(const int32_t* offsets, int n_tiles, int64_t n_isects, cons
 void radix_sort_into(const uint64_t* keys, const int32_t* vals, uint64_t* keys_out, int32_t* vals_out,
                      uint64_t* keys_tmp, int32_t* vals_tmp, int64_t n, uint32_t key_bits, void* scratch,
                      hipStream_t s) {
-    const int passes = static_cast<int>((std::min<uint32_t>(key_bits, 64) + 7) / 8);
+    const int passes = sort_passes<uint64_t>(n, std::min<uint32_t>(key_bits, 64));
     // the last pass, passes - 1, writes side[(passes - 1) & 1]: make that side the output
     uint64_t* const sk[2] = {(passes & 1) ? keys_out : keys_tmp, (passes & 1) ? keys_tmp : keys_out};
     int32_t* const sv[2] = {(passes & 1) ? vals_out : vals_tmp, (passes & 1) ? vals_tmp : vals_out};

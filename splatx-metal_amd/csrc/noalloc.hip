@@ -4,8 +4,8 @@
 // the inputs and outputs are the caller's device buffers, and everything else the sort needs — its
 // histogram/status/error words and the second ping-pong side of the keys and values — lives in the
 // file-scope `scratch` array below, sized for at most kNoAllocMaxKeys keys. Each device the library
-// runs on holds its own copy of the array until the process ends. The sort itself is the onesweep
-// radix sort of sort_isect (k_sort.hip); it clears the words that must start at zero at the start of
+// runs on holds its own copy of the array until the process ends. The sort itself is the
+// radix sort of sort_isect (k_sort.hip); it clears the words that must start at zero in
 // every call, so the array's left-over contents never matter. Calls on one device share the array, so
 // a per-device mutex is held across each call: calls from several host threads are serialised, not
 // raced (work the caller queued on other streams that reads the outputs must wait for the return).
@@ -22,7 +22,7 @@
 namespace {
 
 constexpr int64_t kNoAllocMaxKeys = int64_t{1} << 21;  // 2,097,152 keys
-constexpr size_t kSortRegion = size_t{2} << 20;        // the sort's words for kNoAllocMaxKeys keys (1.02 MiB used)
+constexpr size_t kSortRegion = size_t{2} << 20;        // the sort's words for kNoAllocMaxKeys keys (1.6 MiB used)
 constexpr size_t kKeysRegion = sizeof(uint64_t) * kNoAllocMaxKeys;
 constexpr size_t kValsRegion = sizeof(int32_t) * kNoAllocMaxKeys;
 constexpr size_t kScratchBytes = kSortRegion + kKeysRegion + kValsRegion;  // 26 MiB
@@ -124,8 +124,6 @@ extern "C" int32_t sxh_sort_isect_noalloc(sxh_backend* b, const uint64_t* keys, 
         hipStream_t s = b->stream;
         sxk::radix_sort_into(keys, values, keys_sorted, values_sorted, keys_tmp, vals_tmp, n, key_n_bits, base, s);
         SXH_HIP(hipGetLastError());
-        SXH_HIP(hipMemcpyAsync(b->pinned_word, sxk::sort_error_flag(base), 4, hipMemcpyDeviceToHost, s));
         SXH_HIP(hipStreamSynchronize(s));
-        if (*b->pinned_word) throw std::runtime_error("sort_isect_noalloc: radix sort look-back did not complete");
     });
 }

@@ -293,7 +293,6 @@ struct sxh_backend {
     int device = 0;
     hipStream_t stream = nullptr;
     std::string name;
-    uint32_t* pinned_word = nullptr;  // a pinned host word for status readbacks of the allocation-free calls
     std::unique_ptr<sxh::HostXfer> xfer;  // copies of the callers' arrays
     sxh::DevCache cache;                  // the per-op entry points' device buffers
 };

@@ -72,20 +72,25 @@ void scan_i32_i64(const int32_t* in, int64_t* out, int64_t n, void* scratch, hip
 // lands in keys_a/vals_a when the pass count is even, else in keys_b/vals_b; returns 0 or 1
 // accordingly. The scratch needs sort_scratch_bytes(n) bytes for n keys. With n_dev the key count is
 // read on the device from *n_dev (<= n, which then only sizes the grids; n < 2^30, else -1 is
-// returned and nothing is launched): the launches no longer depend on the count. no_wait (u32 keys and
-// the position sorts): every pass counts its tiles' digits and scans the counts (reduce-then-scan) at
-// any size, so no workgroup waits on another and the sort cannot give up (below 16 tiles of 4096 keys
-// the default onesweep passes wait on their predecessors with a bounded spin).
+// returned and nothing is launched): the launches no longer depend on the count. No workgroup waits on another in any
+// of the sorts.
 size_t sort_scratch_bytes(int64_t n);
 int radix_sort(uint64_t* keys_a, int32_t* vals_a, uint64_t* keys_b, int32_t* vals_b, int64_t n,
                uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                const int64_t* n_dev = nullptr);
 int radix_sort(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n,
                uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
-               const int64_t* n_dev = nullptr, bool no_wait = false);
+               const int64_t* n_dev = nullptr);
 int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                const int64_t* n_dev = nullptr);
+// Where each key value starts in the sorted keys (the number of smaller keys), for values below n: a sort of
+// one pass (at most eight bits) knows it and writes it to starts; `written` says whether it did.
+struct DigitStarts {
+    int32_t* starts;
+    int n;
+    bool written;
+};
 // The same sort with each key's input position as its value (vals_a is not read; the sorted values
 // are the positions of the keys in the unsorted array). x_a (optional, then x_b too): a u32 per key
 // that moves with it, sorted into x_a or x_b like the keys (x_a is the input and, after an even pass
@@ -93,20 +98,19 @@ int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* val
 int radix_sort_positions(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                          const int64_t* n_dev = nullptr, uint32_t* x_a = nullptr, uint32_t* x_b = nullptr,
-                         bool no_wait = false);
+                         DigitStarts* ds = nullptr);
 int radix_sort_positions(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                          const int64_t* n_dev = nullptr, uint32_t* x_a = nullptr, uint32_t* x_b = nullptr,
-                         bool no_wait = false);
+                         DigitStarts* ds = nullptr);
 // The same sort of n u64 keys from read-only inputs into keys_out/vals_out, with keys_tmp/vals_tmp as
-// the second ping-pong side (n > 0, key_bits in 1..64, the onesweep range n < 2^30). No buffer may
+// the second ping-pong side (n > 0, key_bits in 1..64, n < 2^30). No buffer may
 // alias another.
 void radix_sort_into(const uint64_t* keys, const int32_t* vals, uint64_t* keys_out, int32_t* vals_out,
                      uint64_t* keys_tmp, int32_t* vals_tmp, int64_t n, uint32_t key_bits, void* scratch,
                      hipStream_t s);
-// device word in the sort's scratch that a sort sets non-zero when a tile's look-back gave up (a
-// broken invariant, never expected). A sort with clear_err zeroes it first; one without adds to
-// what the sorts before it left, so several sorts in a row can be checked with one read.
+// device word in the sort's scratch that a sort sets non-zero when it could not finish (no path does; callers
+// read it all the same, and a step's test switch sets it). A sort with clear_err zeroes it first.
 uint32_t* sort_error_flag(void* scratch);
 // Equal depths by original row in index-first lists whose Gaussians are numbered in an internal row
 // order: the order of equal depths is row_orig[id_of[value]], and an entry's depth is word 3 of its
