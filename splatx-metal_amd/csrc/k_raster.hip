@@ -346,6 +346,210 @@ __global__ void __launch_bounds__(kThreads) k_raster_fwd(RasterArgs a, float* __
     out_last[pix] = cur;
 }
 
+// ---- forward with a wave per block -----------------------------------------------------------------
+// An image of few tiles leaves the GPU waiting for its heaviest tiles: with four waves a tile, one per SIMD, the
+// walk's dependent chains (list entry, record, exponential, T) are exposed, not issue. Here a tile has sixteen
+// waves, one per 4x4 block, and a wave's four 16-lane groups take four consecutive entries of its block's list:
+// each lane evaluates its own entry's alpha for its pixel, the four alphas are exchanged between the groups
+// (row swaps), and every group runs T through them in list order; group k accumulates colour channel k. The same
+// operations on the same values in the same order as k_raster_fwd, so the same bits; about as many instructions
+// per entry (65 for four entries of one block against 193 for four entries of four blocks walked in lockstep up to
+// the longest list), with four times the waves.
+constexpr int kWideThreads = 1024;
+constexpr int kWideBatch = 512;
+constexpr int kWideRow = kWideBatch + 4;
+constexpr uint32_t kWidePad = kWideBatch * sizeof(float4);
+
+// a[k] = the value of group k (lanes 16 k .. 16 k + 15) at the lane's place in its group
+__device__ __forceinline__ void across_groups(float own, float a[4]) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(own), __float_as_uint(own), false, false);
+    const auto even = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false);  // groups 0 0 2 2 -> 0, 2
+    const auto odd = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false);   // groups 1 1 3 3 -> 1, 3
+    a[0] = __uint_as_float(even[0]);
+    a[2] = __uint_as_float(even[1]);
+    a[1] = __uint_as_float(odd[0]);
+    a[3] = __uint_as_float(odd[1]);
+}
+
+__global__ void __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) k_raster_fwd_wide(RasterArgs a, float* __restrict__ out_rgb,
+                                                                  float* __restrict__ out_alpha,
+                                                                  int32_t* __restrict__ out_last) {
+    __shared__ float4 s_xyo[kWideBatch + 1];  // as in k_raster_fwd, the record no pixel reaches last
+    __shared__ float4 s_con[kWideBatch + 1];
+    __shared__ float4 s_rgb[kWideBatch + 1];
+    __shared__ __align__(16) uint16_t s_list[kBlocks][kWideRow];
+    constexpr int kStageWaves = kWideBatch / 64;
+    __shared__ int s_bc[kBlocks][kStageWaves];
+    __shared__ int s_len[kBlocks];
+    __shared__ unsigned long long s_gen[kStageWaves];
+    const int n_tiles = a.tile_width * a.tile_height;
+    const int img = blockIdx.x / n_tiles;
+    const int tile = a.tile_order ? a.tile_order[blockIdx.x % n_tiles] : static_cast<int>(blockIdx.x % n_tiles);
+    const int tx = tile % a.tile_width, ty = tile / a.tile_width;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, bl = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's block
+    const int grp = lane >> 4, r = lane & 15;
+    const int px_i = tx * 16 + 4 * (bl & 3) + (r & 3), py_i = ty * 16 + 4 * (bl >> 2) + (r >> 2);
+    const bool inside = px_i < a.width && py_i < a.height;
+    const size_t pix = (size_t)img * a.height * a.width + (size_t)py_i * a.width + px_i;
+    const float* bg = a.backgrounds ? a.backgrounds + img * 3 : nullptr;
+    if (a.masks && a.masks[(size_t)img * n_tiles + tile] == 0) {  // uniform per workgroup
+        if (inside) {
+            if (grp < 3) {
+                out_rgb[pix * 3 + grp] = bg ? bg[grp] : 0.f;
+            } else {
+                out_alpha[pix] = 0.f;
+                out_last[pix] = 0;
+            }
+        }
+        return;
+    }
+    const int32_t* offs = a.offsets + (size_t)img * n_tiles;
+    const int32_t range_start = offs[tile];
+    const int32_t range_end = (img == a.I - 1 && tile == n_tiles - 1)
+                                  ? (a.n_isects_dev ? static_cast<int32_t>(*a.n_isects_dev) : a.n_isects)
+                                  : offs[tile + 1];
+    const float px = static_cast<float>(px_i) + 0.5f, py = static_cast<float>(py_i) + 0.5f;
+    float T = 1.0f;    // (the same in every group)
+    int32_t cur = 0;   // the group's own entries: the last one taken
+    float sum = 0.f;   // colour channel grp
+    bool done = !inside;
+    int32_t loaded_end = range_end;
+    if (tid == 0) {
+        s_xyo[kWideBatch] = make_float4(0.f, 0.f, 0.f, -__builtin_inff());
+        s_con[kWideBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_rgb[kWideBatch] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    for (int32_t bstart = range_start; bstart < range_end; bstart += kWideBatch) {
+        if (__syncthreads_count(done) == kWideThreads) {  // also the barrier before LDS reuse
+            loaded_end = bstart;
+            break;
+        }
+        // the first eight waves stage the batch and rank its entries in the blocks' lists (as build_block_lists)
+        uint32_t bm = 0u;
+        if (tid < kWideBatch) {
+            const int32_t idx = bstart + tid;
+            bool odd = false;  // past the polynomial's range, or a colour that a zero weight would not cancel
+            if (idx < range_end) {
+                const int32_t f = a.flatten_ids[idx];
+                const int32_t g = a.id_of ? a.id_of[f] : f;
+                float4 xyo = a.splats[(size_t)g * 3];
+                xyo.w = sigma_cutoff(xyo.z);
+                const float4 con = a.splats[(size_t)g * 3 + 1];
+                const float4 rgb = a.splats[(size_t)g * 3 + 2];
+                s_xyo[tid] = xyo;
+                s_con[tid] = con;
+                s_rgb[tid] = rgb;
+                bm = block_mask(xyo, con, static_cast<float>(tx * 16), static_cast<float>(ty * 16));
+                if (a.block_masks) a.block_masks[idx] = static_cast<uint16_t>(bm);
+                odd = bm != 0u && (xyo.w > 86.0f || !__builtin_isfinite(rgb.x) || !__builtin_isfinite(rgb.y) ||
+                                   !__builtin_isfinite(rgb.z));
+            }
+            const unsigned long long gb = __ballot(odd);
+            if (lane == 0) s_gen[bl] = gb;
+            int cnt = 0;
+#pragma unroll
+            for (int k = 0; k < kBlocks; k++) {
+                const unsigned long long bal = __ballot((bm >> k) & 1u);
+                cnt = lane == k ? __popcll(bal) : cnt;
+            }
+            if (lane < kBlocks) s_bc[lane][bl] = cnt;
+        }
+        __syncthreads();
+        if (tid < kWideBatch) {
+            int off = 0;  // lane k < 16: where the wave's entries of block k start
+            if (lane < kBlocks) {
+                int len = 0;
+#pragma unroll
+                for (int w = 0; w < kStageWaves; w++) {
+                    const int c = s_bc[lane][w];
+                    off += w < bl ? c : 0;
+                    len += c;
+                }
+                if (bl == 0) {
+                    s_len[lane] = len;
+                    for (int q = len; q < ((len + 3) & ~3); q++) s_list[lane][q] = static_cast<uint16_t>(kWidePad);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kBlocks; k++) {
+                const int base = __builtin_amdgcn_readlane(off, k);
+                // (the ballots again: sixteen kept from above would fill the scalar registers)
+                const unsigned long long bal = __ballot((bm >> k) & 1u);
+                const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bal >> 32),
+                                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), 0u)));
+                if ((bm >> k) & 1u) s_list[k][base + rank] = static_cast<uint16_t>(tid * sizeof(float4));
+            }
+        }
+        __syncthreads();
+        unsigned long long any_odd = 0ull;
+#pragma unroll
+        for (int w = 0; w < kStageWaves; w++) any_odd |= s_gen[w];
+        const int len = __builtin_amdgcn_readfirstlane(s_len[bl]);
+        const char* const lds_xyo = reinterpret_cast<const char*>(s_xyo);
+        const char* const lds_con = reinterpret_cast<const char*>(s_con);
+        const char* const lds_chan = reinterpret_cast<const char*>(s_rgb) + 4 * grp;  // (group 3: the record's last word)
+        auto walk = [&](auto odd_batch) {
+            for (int j = 0; j < len; j += 4) {
+                if (__all(done)) break;  // uniform
+                const uint2 pk = *reinterpret_cast<const uint2*>(&s_list[bl][j]);
+                const int off4[4] = {static_cast<int>(pk.x & 0xFFFFu), static_cast<int>(pk.x >> 16),
+                                     static_cast<int>(pk.y & 0xFFFFu), static_cast<int>(pk.y >> 16)};
+                const int off = s_list[bl][j + grp];
+                const float4 xyo = *reinterpret_cast<const float4*>(lds_xyo + off);
+                const float4 con = *reinterpret_cast<const float4*>(lds_con + off);
+                float c4[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) c4[k] = *reinterpret_cast<const float*>(lds_chan + off4[k]);
+                const float sg = sigma_of(con.x, con.y, con.z, xyo.x - px, xyo.y - py);
+                const bool in = !done & !(sg > xyo.w);
+                if (!__any(in)) continue;  // uniform
+                const float vis = decltype(odd_batch)::value ? sxm::expf_fast(-sg) : exp_neg_poly(sg);
+                const float alpha = sxd::smin(sx::kMaxAlpha, xyo.z * vis);
+                const bool ok = in & !(sg < 0.f) & !(alpha < sx::kAlphaThreshold);
+                float own = ok ? alpha : 0.f;  // 0: not taken (T times 1 and the sums unchanged)
+                float al[4], t[5];
+                across_groups(own, al);
+                t[0] = T;
+#pragma unroll
+                for (int k = 0; k < 4; k++) t[k + 1] = t[k] * (1.0f - al[k]);
+                if (__any(t[4] <= sx::kTransmittanceThreshold)) {  // uniform: a lane's T is spent within the chunk
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const float nt = t[k] * (1.0f - al[k]);
+                        done = done | (al[k] > 0.f & nt <= sx::kTransmittanceThreshold);
+                        al[k] = done ? 0.f : al[k];
+                        t[k + 1] = done ? t[k] : nt;
+                    }
+                    own = grp == 0 ? al[0] : grp == 1 ? al[1] : grp == 2 ? al[2] : al[3];
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float w = al[k] * t[k];
+                    if (decltype(odd_batch)::value) sum = al[k] > 0.f ? __builtin_fmaf(c4[k], w, sum) : sum;
+                    else sum = __builtin_fmaf(c4[k], w, sum);
+                }
+                cur = own > 0.f ? bstart + (off >> 4) : cur;
+                T = t[4];
+            }
+        };
+        if (any_odd != 0ull)  // uniform
+            walk(std::true_type{});
+        else
+            walk(std::false_type{});
+    }
+    if (a.block_masks && tid == 0) a.mask_end[(size_t)img * n_tiles + tile] = loaded_end;
+    cur = max(cur, __shfl_xor(cur, 16, 64));
+    cur = max(cur, __shfl_xor(cur, 32, 64));
+    if (!inside) return;
+    if (grp < 3) {
+        out_rgb[pix * 3 + grp] = bg ? __builtin_fmaf(T, bg[grp], sum) : sum;
+    } else {
+        out_alpha[pix] = 1.0f - T;
+        out_last[pix] = cur;
+    }
+}
+
 // ---- group reductions ------------------------------------------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -1124,11 +1328,19 @@ void raster_tile_order(const int32_t* offsets, int n_tiles, int64_t n_isects, in
                        max_count);
 }
 
+// Up to this many tiles a tile gets a wave per block: the GPU holds two such workgroups per compute unit (64 VGPRs),
+// so all of them run at once. Measured, four waves a tile and sixteen: 260 tiles of 2 thousand entries 121 and 73 us,
+// of 4 thousand 258 and 145, 256 tiles of 200 entries 26 and 17, 512 tiles of large splats (every block reached) 39
+// and 41; past 512, where a second round begins, 544 tiles of large splats 40 and 48.
+constexpr int kWideTiles = 512;
+
 void raster_fwd(const RasterArgs& a, float* rgb, float* alpha, int32_t* last, hipStream_t s) {
     const int blocks = a.I * a.tile_width * a.tile_height;
     if (blocks <= 0) return;
     if (a.stats)
         hipLaunchKernelGGL(k_raster_fwd<true>, dim3(blocks), dim3(kThreads), 0, s, a, rgb, alpha, last);
+    else if (blocks <= kWideTiles)
+        hipLaunchKernelGGL(k_raster_fwd_wide, dim3(blocks), dim3(kWideThreads), 0, s, a, rgb, alpha, last);
     else
         hipLaunchKernelGGL(k_raster_fwd<false>, dim3(blocks), dim3(kThreads), 0, s, a, rgb, alpha, last);
 }

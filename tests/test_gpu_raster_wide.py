@@ -1,0 +1,63 @@
+"""The rasterisers on images of few tiles (a wave per 4x4 pixel block) and around the tile count where they change to
+four waves a tile (512): lists around the batch (512 entries) and chunk (4) edges, where a pixel's transmittance is
+spent within a chunk, colours that a zero weight would not cancel, masks, backgrounds and several images."""
+import numpy as np
+import pytest
+
+import inputs
+from test_gpu_ops import extreme_splats, rel_l2, same_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def check(gpu, oracle, kw, grads=True):
+    a, b = gpu.rasterize_fwd(**kw), oracle.rasterize_fwd(**kw)
+    for k in ("render_colors", "render_alphas", "last_ids"):
+        assert same_bits(a[k], b[k]), k
+    if not grads:
+        return
+    r = inputs.rng(5)
+    gin = dict(render_alphas=b["render_alphas"], last_ids=b["last_ids"],
+               v_render_colors=r.standard_normal(b["render_colors"].shape).astype(np.float32),
+               v_render_alphas=r.standard_normal(b["render_alphas"].shape).astype(np.float32))
+    ga, gb = gpu.rasterize_bwd(**gin, **kw), oracle.rasterize_bwd(**gin, **kw)
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        assert rel_l2(ga[k], gb[k]) <= 1e-4, (k, rel_l2(ga[k], gb[k]))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 31, 33, 255, 257, 511, 512, 513, 1025])
+def test_list_lengths(gpu, oracle, n):
+    print(f"entries {n}", flush=True)
+    check(gpu, oracle, extreme_splats(50 + n, n=n, width=37, height=21))
+
+
+@pytest.mark.parametrize("size", [(512, 256), (513, 256), (432, 304)])  # 512, 528 and 513 tiles
+def test_tile_counts(gpu, oracle, size):
+    print(f"size {size}", flush=True)
+    check(gpu, oracle, extreme_splats(7, n=150, width=size[0], height=size[1]))
+
+
+@pytest.mark.parametrize("opacity", [0.3, 0.9, 0.99])
+def test_spent_within_a_chunk(gpu, oracle, opacity):
+    """Opaque splats over every pixel: T runs out after a number of entries that differs between pixels."""
+    kw = extreme_splats(8, n=600, width=40, height=24)
+    kw["opacities"] = np.full_like(kw["opacities"], opacity)
+    kw["conics"] = np.tile(np.array([0.002, 0.0005, 0.003], np.float32), (1, 600, 1))
+    check(gpu, oracle, kw)
+
+
+def test_colours_not_finite(gpu, oracle):
+    kw = extreme_splats(9, n=300, width=48, height=32)
+    c = kw["colors"].copy()
+    c[0, 10:40:6, 0], c[0, 12:60:9, 1], c[0, 11:60:4, 2] = np.inf, -np.inf, np.nan
+    kw["colors"] = c
+    a, b = gpu.rasterize_fwd(**kw), oracle.rasterize_fwd(**kw)
+    assert same_bits(a["render_alphas"], b["render_alphas"]) and same_bits(a["last_ids"], b["last_ids"])
+    x, y = a["render_colors"], b["render_colors"]
+    assert np.isnan(y).any() and np.isinf(y).any() and np.isfinite(y).any()
+    assert np.array_equal(np.isnan(x), np.isnan(y))
+    assert same_bits(np.nan_to_num(x, nan=0.0), np.nan_to_num(y, nan=0.0))
+
+
+def test_images_masks_backgrounds(gpu, oracle):
+    check(gpu, oracle, inputs.raster_kwargs(oracle, n=900, seed=11, I=2, width=75, height=45, backgrounds=True, masks=True))
