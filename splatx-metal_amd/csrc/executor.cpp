@@ -410,7 +410,10 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
     volatile unsigned long long* const hc = static_cast<volatile unsigned long long*>(e->step_rb.p);
     volatile uint32_t* const hw = reinterpret_cast<volatile uint32_t*>(hc + 2);
     unsigned long long seq = 0;  // the last segment A's sequence number (its count word's tag)
-    auto launch_a = [&](unsigned long long cap) {
+    // fold: the block scan rides on the emit's launch, at the head of segment B
+    const bool can_fold = index_first && sxk::step_preprocess_blocks(c.count) <= sxk::kFoldBlocks;
+    sxk::EmitFold fold;
+    auto launch_a = [&](unsigned long long cap, bool folded) {
         seq = ++e->step_seq;
         if (e->prof_stats)
             SXH_HIP(hipMemsetAsync(e->rstats.p, 0, sxk::kRasterStats * sizeof(unsigned long long), s));
@@ -424,14 +427,18 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                                         sxk::sort_error_flag(e->sort_scratch.p), e->radii.p, e->tiles.p,
                                         e->vis_part.p, e->n_vis.p, e->blk_base.p, cap,
                                         static_cast<unsigned long long*>(e->step_rb.dev), seq, clr, s, row_orig,
-                                        row_int, e->tiles_o.p);
+                                        row_int, e->tiles_o.p, folded);
             e->mark("update_preprocess");
         } else {
             sxk::step_preprocess(c, A, e->splats.p, e->radii.p, e->tiles.p, e->vis_part.p, e->n_vis.p, e->blk_base.p,
                                  cap, static_cast<unsigned long long*>(e->step_rb.dev), seq, clr, s, row_int,
-                                 e->tiles_o.p);
+                                 e->tiles_o.p, folded);
             e->mark("preprocess");
         }
+        fold = sxk::EmitFold{};
+        if (folded)
+            fold = {reinterpret_cast<const uint4*>(e->vis_part.p), sxk::step_preprocess_blocks(c.count), cap, e->n_vis.p,
+                    static_cast<unsigned long long*>(e->step_rb.dev), seq};
     };
     const float* gt = nullptr;
     auto upload_gt = [&]() {
@@ -483,35 +490,42 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         uint32_t* const edepth_b =
             index_first ? reinterpret_cast<uint32_t*>(e->keys_a.p) + e->isect_cap : nullptr;
         int which = 0;
-        sxk::DigitStarts starts{e->offsets.p, n_tiles, false};  // (up to 256 tiles the sort leaves the offsets)
+        // (up to 256 tiles the sort leaves the offsets; the emit clears the words the sort adds into)
+        sxk::SortExtra extra{e->offsets.p, n_tiles, false, false};
+        sxk::EmitZero zero;
+        if (c.tile_n_bits <= 16) {
+            const sxk::SortZeroWords z = sxk::sort_zero_words_u16(e->sort_scratch.p, n_host);
+            zero = {z.words, z.n};
+            extra.zeroed = true;
+        }
         if (c.tile_n_bits <= 16) {
             uint16_t* ka = reinterpret_cast<uint16_t*>(e->keys_a.p);
             uint16_t* kb = reinterpret_cast<uint16_t*>(e->keys_b.p);
             if (index_first)
                 sxk::step_emit_compact_sorted(c, e->splats.p, e->radii.p, e->tiles.p, e->blk_base.p, e->emit_list.p,
-                                              e->cum.p, n_emit, ka, e->emit_gid.p, s, edepth);
+                                              e->cum.p, n_emit, ka, e->emit_gid.p, s, edepth, fold, zero);
             else
                 sxk::step_emit_sorted(c, e->splats.p, e->radii.p, order, e->cum.p, n_emit, ka, e->emit_gid.p, s,
-                                      edepth);
+                                      edepth, zero);
             e->mark("emit");
             which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
-                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &starts);
+                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &extra);
             e->mark("sort");
-            if (!starts.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
+            if (!extra.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
         } else {
             uint32_t* ka = reinterpret_cast<uint32_t*>(e->keys_a.p);
             uint32_t* kb = reinterpret_cast<uint32_t*>(e->keys_b.p);
             if (index_first)
                 sxk::step_emit_compact_sorted(c, e->splats.p, e->radii.p, e->tiles.p, e->blk_base.p, e->emit_list.p,
-                                              e->cum.p, n_emit, ka, e->emit_gid.p, s, edepth);
+                                              e->cum.p, n_emit, ka, e->emit_gid.p, s, edepth, fold, zero);
             else
                 sxk::step_emit_sorted(c, e->splats.p, e->radii.p, order, e->cum.p, n_emit, ka, e->emit_gid.p, s,
-                                      edepth);
+                                      edepth, zero);
             e->mark("emit");
             which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
-                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &starts);
+                                              e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &extra);
             e->mark("sort");
-            if (!starts.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
+            if (!extra.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
         }
         if (which < 0) throw std::runtime_error(std::string(what) + ": intersection capacity too large for a device count");
         if (e->debug_sort_error) sxk::step_set_word(sxk::sort_error_flag(e->sort_scratch.p), 1u, s);
@@ -660,7 +674,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
     e->sync_ms[0] = 0.0;
     if (graph_ok()) {
         const unsigned long long cap = e->isect_cap;
-        launch_a(cap);
+        launch_a(cap, can_fold);
         upload_gt();
         capture_b();
         SXH_HIP(hipGraphLaunch(e->graph_b[index_first ? 1 : 0][fwd_only ? 1 : 0], s));
@@ -676,7 +690,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         upload_gt();
     }
     if (!done) {
-        launch_a(~0ull);
+        launch_a(~0ull, false);
         const auto t0 = std::chrono::steady_clock::now();
         SXH_HIP(hipStreamSynchronize(s));
         e->sync_ms[0] += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

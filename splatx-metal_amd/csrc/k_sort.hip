@@ -777,7 +777,7 @@ int sort_passes(int64_t n, uint32_t key_bits) {
 template <class K>
 int radix_sort_t(const K* src_k, const int32_t* src_v, K* const side_k[2], int32_t* const side_v[2], int64_t n,
                  uint32_t key_bits, void* scratch, bool clear_err, hipStream_t s, const int64_t* n_dev,
-                 const uint32_t* src_x = nullptr, uint32_t* const* side_x = nullptr, DigitStarts* ds = nullptr) {
+                 const uint32_t* src_x = nullptr, uint32_t* const* side_x = nullptr, SortExtra* ds = nullptr) {
     uint32_t* totals = static_cast<uint32_t*>(scratch);
     uint32_t* err = totals + kErrWord;
     key_bits = std::min<uint32_t>(key_bits, 8 * sizeof(K));
@@ -802,7 +802,7 @@ int radix_sort_t(const K* src_k, const int32_t* src_v, K* const side_k[2], int32
         uint32_t* const cnt = hist;
         // the passes' group sums in turn: a pass's count clears the next one's
         uint32_t* const gs[2] = {cnt + (size_t)rows.tiles * T, cnt + (size_t)(rows.tiles + rows.groups) * T};
-        if (rows.groups)
+        if (rows.groups && !(ds && ds->zeroed))
             hipLaunchKernelGGL(k_zero_words, dim3((rows.groups * T + kThreads - 1) / kThreads), dim3(kThreads), 0, s, gs[0],
                                rows.groups * T);
         if (ds) ds->written = passes == 1;
@@ -897,7 +897,7 @@ int radix_sort_t(const K* src_k, const int32_t* src_v, K* const side_k[2], int32
 template <class K>
 int radix_sort_ab(K* keys_a, int32_t* vals_a, K* keys_b, int32_t* vals_b, int64_t n, uint32_t key_bits,
                   void* scratch, bool clear_err, hipStream_t s, const int64_t* n_dev, bool index_values = false,
-                  uint32_t* x_a = nullptr, uint32_t* x_b = nullptr, DigitStarts* ds = nullptr) {
+                  uint32_t* x_a = nullptr, uint32_t* x_b = nullptr, SortExtra* ds = nullptr) {
     K* const sk[2] = {keys_b, keys_a};
     int32_t* const sv[2] = {vals_b, vals_a};
     uint32_t* const sx[2] = {x_b, x_a};
@@ -1305,6 +1305,13 @@ k_tile_depth_sort(const int32_t* __restrict__ offsets, int n_tiles, int32_t n_is
 
 } // namespace
 
+SortZeroWords sort_zero_words_u16(void* scratch, int64_t n) {
+    using Plan = RowPlan<uint16_t>;
+    const Plan rows(n);
+    if (!rows.fits || rows.groups == 0) return {nullptr, 0};
+    return {static_cast<uint32_t*>(scratch) + kHeaderWords + (size_t)rows.tiles * Plan::kT, rows.groups * Plan::kT};
+}
+
 size_t sort_scratch_bytes(int64_t n) {
     const size_t tiles = static_cast<size_t>(std::max(1, tiles_for(n)));
     size_t words = 2 * tiles * kBins;
@@ -1334,13 +1341,13 @@ int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* val
 
 int radix_sort_positions(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev,
-                         uint32_t* x_a, uint32_t* x_b, DigitStarts* ds) {
+                         uint32_t* x_a, uint32_t* x_b, SortExtra* ds) {
     return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b, ds);
 }
 
 int radix_sort_positions(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err, const int64_t* n_dev,
-                         uint32_t* x_a, uint32_t* x_b, DigitStarts* ds) {
+                         uint32_t* x_a, uint32_t* x_b, SortExtra* ds) {
     return radix_sort_ab(keys_a, vals_a, keys_b, vals_b, n, key_bits, scratch, clear_err, s, n_dev, true, x_a, x_b, ds);
 }
 

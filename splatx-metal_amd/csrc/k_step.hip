@@ -419,6 +419,51 @@ __device__ __forceinline__ sxd::F2 line_upper_cut(const sxd::AccuSweep& sw, int 
     return sxd::accutile_start(sw);
 }
 
+// The block scan (k_block_scan) in the emit's own launch, for up to kFoldBlocks preprocess blocks: every workgroup adds
+// up the counts of the blocks before its own and of all (16 B each, 16 KB at most, from L2), and the first one
+// leaves the totals where k_block_scan does. Saves a launch of one workgroup, 5 us of a step of 115 to 380.
+__device__ __forceinline__ void fold_block_scan(const EmitFold& f, unsigned long long& base_i, unsigned long long& base_e,
+                                                unsigned long long& n_all) {
+    __shared__ unsigned long long s_sum[kBlock / 64][5];
+    unsigned long long v[5] = {0, 0, 0, 0, 0};  // before: intersections, Gaussians with tiles; all: those, visible
+    for (int b = threadIdx.x; b < f.n_blocks; b += kBlock) {
+        const uint4 p = f.part[b];
+        const bool before = b < static_cast<int>(blockIdx.x);
+        v[0] += before ? p.y : 0u;
+        v[1] += before ? p.z : 0u;
+        v[2] += p.y;
+        v[3] += p.z;
+        v[4] += p.x;
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+        if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6][k] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        v[k] = 0;
+#pragma unroll
+        for (int w = 0; w < kBlock / 64; w++) v[k] += s_sum[w][k];
+    }
+    const bool ovf = v[2] > f.cap;
+    base_i = v[0];
+    base_e = v[1];
+    n_all = ovf ? 0ull : v[3];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        f.out[0] = v[4];
+        f.out[1] = v[2];
+        f.out[2] = n_all;
+        f.out[3] = ovf ? 0ull : v[2];
+        f.out[4] = ovf ? 1ull : 0ull;
+        store_host(&f.host[0], v[4]);
+        store_host(&f.host[1], v[2]);
+        __hip_atomic_store(&f.host[4], f.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // COMPACT (index order): the workgroup takes the 256 rows of preprocess block b instead of 256 emit
 // positions, and compacts them first as k_emit_compact does (tiles: the rows' tile counts, base: the block
 // scan's bases), writing the list and the offsets (list, cum_out) for the later kernels; a lane's
@@ -432,8 +477,11 @@ __global__ void __launch_bounds__(kBlock) k_emit_sorted(StepConst c, const float
                                                         const unsigned long long* __restrict__ n_pos,
                                                         const int32_t* __restrict__ tiles,
                                                         const unsigned long long* __restrict__ base,
-                                                        int32_t* __restrict__ list, int64_t* __restrict__ cum_out) {
+                                                        int32_t* __restrict__ list, int64_t* __restrict__ cum_out,
+                                                        EmitFold fold, EmitZero zero) {
     __shared__ EmitWave s_w[kBlock / 64];
+    // words that a later kernel of the step adds into, cleared here
+    for (int q = blockIdx.x * kBlock + threadIdx.x; q < zero.n; q += gridDim.x * kBlock) zero.words[q] = 0u;
     const int j = blockIdx.x * kBlock + threadIdx.x;
     const int lane = threadIdx.x & 63;
     EmitWave& W = s_w[threadIdx.x >> 6];
@@ -469,9 +517,17 @@ __global__ void __launch_bounds__(kBlock) k_emit_sorted(StepConst c, const float
                 pn += s_n[w];
                 pt += s_t[w];
             }
-        const unsigned long long jj = base[2 * (size_t)blockIdx.x + 1] + pn + rank;
-        if (t > 0u && jj < *n_pos) {  // (n_pos reads 0 after an overflow: nothing is written)
-            const int64_t end = static_cast<int64_t>(base[2 * (size_t)blockIdx.x] + pt + incl);
+        unsigned long long base_i, base_e, n_all;  // intersections and Gaussians with tiles before the block, the latter in all
+        if (fold.part) {
+            fold_block_scan(fold, base_i, base_e, n_all);
+        } else {
+            base_i = base[2 * (size_t)blockIdx.x];
+            base_e = base[2 * (size_t)blockIdx.x + 1];
+            n_all = *n_pos;
+        }
+        const unsigned long long jj = base_e + pn + rank;
+        if (t > 0u && jj < n_all) {  // (0 after an overflow: nothing is written)
+            const int64_t end = static_cast<int64_t>(base_i + pt + incl);
             list[jj] = j;
             cum_out[jj] = end;
             my0 = end - t;
@@ -891,7 +947,7 @@ __global__ void k_step_readback(StepReadback rb) {
 void step_preprocess(const StepConst& c, const Arena& A, float4* splats, int32_t* radii, int32_t* tiles,
                      uint32_t* vis_part, unsigned long long* n_visible, unsigned long long* block_base,
                      unsigned long long isect_cap, unsigned long long* host_counts, unsigned long long seq,
-                     const StepClear& clr, hipStream_t s, const int32_t* row_int, int32_t* tiles_o) {
+                     const StepClear& clr, hipStream_t s, const int32_t* row_int, int32_t* tiles_o, bool fold_scan) {
     if (c.count <= 0) return;
     const dim3 grid(grid_for(c.count)), block(kBlock);
     switch (c.n_coeffs) {
@@ -903,8 +959,9 @@ void step_preprocess(const StepConst& c, const Arena& A, float4* splats, int32_t
     }
     if (row_int)  // the tile counts and the block counts in original order
         hipLaunchKernelGGL(k_orig_block_counts, grid, block, 0, s, row_int, c.count, tiles, tiles_o, vis_part);
-    hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanBlock), 0, s, reinterpret_cast<const uint4*>(vis_part),
-                       static_cast<int>(grid.x), n_visible, block_base, isect_cap, host_counts, seq);
+    if (!fold_scan)
+        hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanBlock), 0, s, reinterpret_cast<const uint4*>(vis_part),
+                           static_cast<int>(grid.x), n_visible, block_base, isect_cap, host_counts, seq);
 }
 
 void step_emit_compact(const StepConst& c, const int32_t* tiles, const unsigned long long* block_base, int32_t* list,
@@ -925,42 +982,42 @@ void step_depth_keys(const StepConst& c, const float4* splats, const int32_t* li
 
 void step_emit_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* order,
                       const int64_t* cum, const unsigned long long* n_pos, uint16_t* keys, int32_t* vals,
-                      hipStream_t s, uint32_t* edepth) {
+                      hipStream_t s, uint32_t* edepth, const EmitZero& zero) {
     if (c.count <= 0) return;
     hipLaunchKernelGGL((k_emit_sorted<uint16_t, false>), dim3(grid_for(c.count)), dim3(kBlock), 0, s, c, splats, radii,
-                       order, cum, keys, vals, edepth, n_pos, nullptr, nullptr, nullptr, nullptr);
+                       order, cum, keys, vals, edepth, n_pos, nullptr, nullptr, nullptr, nullptr, EmitFold{}, zero);
 }
 
 void step_emit_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* order,
                       const int64_t* cum, const unsigned long long* n_pos, uint32_t* keys, int32_t* vals,
-                      hipStream_t s, uint32_t* edepth) {
+                      hipStream_t s, uint32_t* edepth, const EmitZero& zero) {
     if (c.count <= 0) return;
     hipLaunchKernelGGL((k_emit_sorted<uint32_t, false>), dim3(grid_for(c.count)), dim3(kBlock), 0, s, c, splats, radii,
-                       order, cum, keys, vals, edepth, n_pos, nullptr, nullptr, nullptr, nullptr);
+                       order, cum, keys, vals, edepth, n_pos, nullptr, nullptr, nullptr, nullptr, EmitFold{}, zero);
 }
 
 template <class K>
 static void launch_emit_compact_sorted(const StepConst& c, const float4* splats, const int32_t* radii,
                                        const int32_t* tiles, const unsigned long long* block_base, int32_t* list,
                                        int64_t* cum, const unsigned long long* n_pos, K* keys, int32_t* vals,
-                                       hipStream_t s, uint32_t* edepth) {
+                                       hipStream_t s, uint32_t* edepth, const EmitFold& fold, const EmitZero& zero) {
     if (c.count <= 0) return;
     hipLaunchKernelGGL((k_emit_sorted<K, true>), dim3(grid_for(c.count)), dim3(kBlock), 0, s, c, splats, radii,
-                       nullptr, nullptr, keys, vals, edepth, n_pos, tiles, block_base, list, cum);
+                       nullptr, nullptr, keys, vals, edepth, n_pos, tiles, block_base, list, cum, fold, zero);
 }
 
 void step_emit_compact_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* tiles,
                               const unsigned long long* block_base, int32_t* list, int64_t* cum,
                               const unsigned long long* n_pos, uint16_t* keys, int32_t* vals, hipStream_t s,
-                              uint32_t* edepth) {
-    launch_emit_compact_sorted(c, splats, radii, tiles, block_base, list, cum, n_pos, keys, vals, s, edepth);
+                              uint32_t* edepth, const EmitFold& fold, const EmitZero& zero) {
+    launch_emit_compact_sorted(c, splats, radii, tiles, block_base, list, cum, n_pos, keys, vals, s, edepth, fold, zero);
 }
 
 void step_emit_compact_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* tiles,
                               const unsigned long long* block_base, int32_t* list, int64_t* cum,
                               const unsigned long long* n_pos, uint32_t* keys, int32_t* vals, hipStream_t s,
-                              uint32_t* edepth) {
-    launch_emit_compact_sorted(c, splats, radii, tiles, block_base, list, cum, n_pos, keys, vals, s, edepth);
+                              uint32_t* edepth, const EmitFold& fold, const EmitZero& zero) {
+    launch_emit_compact_sorted(c, splats, radii, tiles, block_base, list, cum, n_pos, keys, vals, s, edepth, fold, zero);
 }
 
 // n (the count, or with n_dev its upper bound) picks the way: the pass up to 2^25 ids
@@ -994,7 +1051,7 @@ void step_update_preprocess(const StepConst& cu, const StepConst& c, const Arena
                             int32_t* tiles, uint32_t* vis_part, unsigned long long* n_visible,
                             unsigned long long* block_base, unsigned long long isect_cap, unsigned long long* host_counts,
                             unsigned long long seq, const StepClear& clr, hipStream_t s, const int32_t* row_orig,
-                            const int32_t* row_int, int32_t* tiles_o) {
+                            const int32_t* row_int, int32_t* tiles_o, bool fold_scan) {
     if (c.count <= 0) return;
     if (cu.count != c.count || cu.n_coeffs != c.n_coeffs)
         throw std::invalid_argument("update_preprocess: both steps must cover the same rows");
@@ -1014,8 +1071,9 @@ void step_update_preprocess(const StepConst& cu, const StepConst& c, const Arena
 #undef SX_UPD
     if (row_int)  // the tile counts and the block counts in original order
         hipLaunchKernelGGL(k_orig_block_counts, grid, block, 0, s, row_int, c.count, tiles, tiles_o, vis_part);
-    hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanBlock), 0, s, reinterpret_cast<const uint4*>(vis_part),
-                       static_cast<int>(grid.x), n_visible, block_base, isect_cap, host_counts, seq);
+    if (!fold_scan)
+        hipLaunchKernelGGL(k_block_scan, dim3(1), dim3(kScanBlock), 0, s, reinterpret_cast<const uint4*>(vis_part),
+                           static_cast<int>(grid.x), n_visible, block_base, isect_cap, host_counts, seq);
 }
 
 void step_postprocess(const StepConst& c, const Arena& A, const float4* splats, const float4* grads,

@@ -84,13 +84,21 @@ int radix_sort(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* val
 int radix_sort(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                const int64_t* n_dev = nullptr);
-// Where each key value starts in the sorted keys (the number of smaller keys), for values below n: a sort of
-// one pass (at most eight bits) knows it and writes it to starts; `written` says whether it did.
-struct DigitStarts {
+// What a caller of a u16 position sort can take off it. starts (optional): where each key value below n starts in
+// the sorted keys (the number of smaller keys); a sort of one pass (at most eight bits) knows it and writes it
+// there, and sets `written`. zeroed: the caller has cleared the words of sort_zero_words on the stream.
+struct SortExtra {
     int32_t* starts;
     int n;
+    bool zeroed;
     bool written;
 };
+// The words that a u16 sort of n keys adds into and needs cleared before its first launch (n: 0 if none).
+struct SortZeroWords {
+    uint32_t* words;
+    int n;
+};
+SortZeroWords sort_zero_words_u16(void* scratch, int64_t n);
 // The same sort with each key's input position as its value (vals_a is not read; the sorted values
 // are the positions of the keys in the unsorted array). x_a (optional, then x_b too): a u32 per key
 // that moves with it, sorted into x_a or x_b like the keys (x_a is the input and, after an even pass
@@ -98,11 +106,11 @@ struct DigitStarts {
 int radix_sort_positions(uint16_t* keys_a, int32_t* vals_a, uint16_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                          const int64_t* n_dev = nullptr, uint32_t* x_a = nullptr, uint32_t* x_b = nullptr,
-                         DigitStarts* ds = nullptr);
+                         SortExtra* extra = nullptr);
 int radix_sort_positions(uint32_t* keys_a, int32_t* vals_a, uint32_t* keys_b, int32_t* vals_b, int64_t n,
                          uint32_t key_bits, void* scratch, hipStream_t s, bool clear_err = true,
                          const int64_t* n_dev = nullptr, uint32_t* x_a = nullptr, uint32_t* x_b = nullptr,
-                         DigitStarts* ds = nullptr);
+                         SortExtra* extra = nullptr);
 // The same sort of n u64 keys from read-only inputs into keys_out/vals_out, with keys_tmp/vals_tmp as
 // the second ping-pong side (n > 0, key_bits in 1..64, n < 2^30). No buffer may
 // alias another.

@@ -67,7 +67,23 @@ void step_preprocess(const StepConst& c, const Arena& A, float4* splats, int32_t
                      uint32_t* vis_part, unsigned long long* out_vis, unsigned long long* block_base,
                      unsigned long long isect_cap, unsigned long long* host_counts, unsigned long long seq,
                      const StepClear& clr, hipStream_t s, const int32_t* row_int = nullptr,
-                     int32_t* tiles_o = nullptr);
+                     int32_t* tiles_o = nullptr, bool fold_scan = false);
+// fold_scan: no block scan after the preprocess; the emit that follows (step_emit_compact_sorted) does it, from this
+// launch's counts. For at most kFoldBlocks blocks.
+struct EmitFold {
+    const uint4* part = nullptr;  // the preprocess blocks' counts (vis_part)
+    int n_blocks = 0;
+    unsigned long long cap = 0;           // isect_cap, out_vis, host_counts and seq of step_preprocess
+    unsigned long long* out = nullptr;
+    unsigned long long* host = nullptr;
+    unsigned long long seq = 0;
+};
+constexpr int kFoldBlocks = 1024;  // 262,144 rows: 16 KB of counts read by every workgroup of the emit
+// Words cleared by the emit's launch for a later kernel of the step.
+struct EmitZero {
+    uint32_t* words = nullptr;
+    int n = 0;
+};
 // number of blocks of step_preprocess
 int step_preprocess_blocks(int64_t count);
 // The Gaussians with tiles in index order (list[j], j below out_vis[2]) and (cum set) cum[j], the
@@ -87,10 +103,10 @@ void step_depth_keys(const StepConst& c, const float4* splats, const int32_t* li
                      uint32_t* keys, int32_t* vals, hipStream_t s);
 void step_emit_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* order,
                       const int64_t* cum, const unsigned long long* n_pos, uint16_t* keys, int32_t* vals,
-                      hipStream_t s, uint32_t* edepth = nullptr);
+                      hipStream_t s, uint32_t* edepth = nullptr, const EmitZero& zero = {});
 void step_emit_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* order,
                       const int64_t* cum, const unsigned long long* n_pos, uint32_t* keys, int32_t* vals,
-                      hipStream_t s, uint32_t* edepth = nullptr);
+                      hipStream_t s, uint32_t* edepth = nullptr, const EmitZero& zero = {});
 // Index first in one launch: step_emit_compact (without row_int) and step_emit_sorted over its list
 // (order = the list): each workgroup compacts the 256 rows of one preprocess block, writes their list
 // entries and offsets (list, cum: for the gather) and emits their tile ids; *n_pos (the count of
@@ -98,11 +114,11 @@ void step_emit_sorted(const StepConst& c, const float4* splats, const int32_t* r
 void step_emit_compact_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* tiles,
                               const unsigned long long* block_base, int32_t* list, int64_t* cum,
                               const unsigned long long* n_pos, uint16_t* keys, int32_t* vals, hipStream_t s,
-                              uint32_t* edepth);
+                              uint32_t* edepth, const EmitFold& fold = {}, const EmitZero& zero = {});
 void step_emit_compact_sorted(const StepConst& c, const float4* splats, const int32_t* radii, const int32_t* tiles,
                               const unsigned long long* block_base, int32_t* list, int64_t* cum,
                               const unsigned long long* n_pos, uint32_t* keys, int32_t* vals, hipStream_t s,
-                              uint32_t* edepth);
+                              uint32_t* edepth, const EmitFold& fold = {}, const EmitZero& zero = {});
 // n_dev: the key count on the device, read instead of n
 void step_tile_offsets(const uint16_t* keys, int64_t n, int n_tiles, int32_t* offsets, hipStream_t s,
                        const int64_t* n_dev = nullptr);
@@ -149,7 +165,7 @@ void step_update_preprocess(const StepConst& cu, const StepConst& c, const Arena
                             unsigned long long* block_base, unsigned long long isect_cap, unsigned long long* host_counts,
                             unsigned long long seq, const StepClear& clr, hipStream_t s,
                             const int32_t* row_orig = nullptr, const int32_t* row_int = nullptr,
-                            int32_t* tiles_o = nullptr);
+                            int32_t* tiles_o = nullptr, bool fold_scan = false);
 // The arena's spatial order (row_orig[k]: the original row of internal row k; row_int its inverse;
 // nothing is reordered past the live rows [0, count)). arena_morton_keys: keys[i] = the 30-bit Morton
 // code of row i's mean in the means' bounding box, vals[i] = i (scratch: arena_morton_scratch_floats).
