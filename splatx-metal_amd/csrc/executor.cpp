@@ -294,7 +294,7 @@ void sxh_detail::canonicalize(sxh_executor* e) {
 
 // The live rows [0, count) along a Morton curve over their means (the arena in original order, no
 // update pending): keys and a stable sort of them, then every parameter and moment column reordered.
-static void spatial_order(sxh_executor* e, int count) {
+void sxh_detail::spatial_order(sxh_executor* e, int count) {
     hipStream_t s = e->b->stream;
     if (e->row_orig.n < static_cast<size_t>(e->rows)) {
         e->row_orig.alloc(static_cast<size_t>(e->rows));
@@ -376,13 +376,12 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
     const sxk::Arena A = e->arena();
     // the live rows' order: spatial ones cover this step's rows; a cloud that stayed on the device for a
     // step since it last exchanged rows with the caller goes into spatial order (at most a few ms, once)
-    constexpr int kSpatialMinRows = 1 << 16;
     if (e->permuted && e->perm_count != c.count) sxh_detail::canonicalize(e);
     if (!fwd_only && !e->permuted &&
         ((e->row_order == SXH_ROW_ORDER_SPATIAL) ||
-         (e->row_order == SXH_ROW_ORDER_SPATIAL_AUTO && c.count >= kSpatialMinRows && e->steps_since_exchange >= 2))) {
+         (e->row_order == SXH_ROW_ORDER_SPATIAL_AUTO && c.count >= sxh_detail::kSpatialMinRows && e->steps_since_exchange >= 2))) {
         sxh_detail::flush_update(e);
-        spatial_order(e, c.count);
+        sxh_detail::spatial_order(e, c.count);
     }
     // index-first sorts each tile's list by depth in one workgroup: fast while the tiles stay small
     // (up to 2048 entries in LDS, larger ones through global scratch, correct at any size)

@@ -535,6 +535,10 @@ int32_t sxh_render_session_open(sxh_backend* b, const sxh_render_session_args* a
             }
             b->xfer->to_device(items, s);
             SXH_HIP(hipGetLastError());
+            // laid out once for every frame: rows in view share lines, rows out of view are skipped by whole waves (1 M
+            // rows, 1297x840: preprocess 62 -> 49 us, emit 34 -> 25, forward 152 -> 147, per-tile depth sort 31 -> 32;
+            // 60 thousand rows: no difference)
+            if (e->rows >= sxh_detail::kSpatialMinRows) sxh_detail::spatial_order(e, e->rows);
             SXH_HIP(hipStreamSynchronize(s));
         } catch (...) {
             if (sess->e) sxh_exec_destroy(sess->e);

@@ -210,4 +210,8 @@ void flush_update(sxh_executor* e);
 // Before a call exchanges rows with the caller: flush_update, then the arena back in the caller's row
 // order if it is in spatial order. Defined in executor.cpp.
 void canonicalize(sxh_executor* e);
+// The rows [0, count), in original order with no update pending, into spatial order: worth its one pass over the arena
+// from kSpatialMinRows rows on. Defined in executor.cpp.
+constexpr int kSpatialMinRows = 1 << 16;
+void spatial_order(sxh_executor* e, int count);
 }  // namespace sxh_detail
