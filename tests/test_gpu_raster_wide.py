@@ -46,6 +46,16 @@ def test_spent_within_a_chunk(gpu, oracle, opacity):
     check(gpu, oracle, kw)
 
 
+@pytest.mark.parametrize("n", [63, 64, 65, 127, 129, 255, 256, 257, 321])
+def test_backward_segments(gpu, oracle, n):
+    """Faint splats over every pixel: each block's list holds all entries, around the segment (64) and the batch (256)
+    of the backward. The sums run over 16 pixels and 16 blocks in 32 bits, T over n factors: below 1e-4."""
+    kw = extreme_splats(20 + n, n=n, width=33, height=18)
+    kw["opacities"] = np.full_like(kw["opacities"], 0.02)
+    kw["conics"] = np.tile(np.array([0.002, 0.0005, 0.003], np.float32), (1, n, 1))
+    check(gpu, oracle, kw)
+
+
 def test_colours_not_finite(gpu, oracle):
     kw = extreme_splats(9, n=300, width=48, height=32)
     c = kw["colors"].copy()
