@@ -1083,276 +1083,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
     }
 }
 
-// A value's copies for the lower and the upper of two groups (pair_of: groups 0, 1 and 2, 3), of two halves of the wave
-// (half_of), in every lane of both.
-struct LoHi {
-    float lo, hi;
-};
-__device__ __forceinline__ LoHi pair_of(float v) {
-    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return {__uint_as_float(p[0]), __uint_as_float(p[1])};
-}
-__device__ __forceinline__ LoHi half_of(float v) {
-    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return {__uint_as_float(p[0]), __uint_as_float(p[1])};
-}
-
-// The backward for images of few tiles: sixteen waves a tile, each on one 4x4 block, as in the wide forward. The four
-// groups of a wave hold the block's pixels and take four consecutive entries of its list; T through the group's entry
-// and the back-sum before it are prefixes over the four groups (row swaps), and each group works out its own entry's
-// gradients. Bound: with four waves a tile, the dependent chain of the heaviest tile (348 VALU instructions per four
-// entries, over the longest of four blocks' lists); here about 120 over the block's own list, four waves a SIMD. The
-// exponential is always the forward's: for one entry the test that would allow the hardware's costs as much. The
-// register spills of the staging (15, once per batch) are cheaper than half the workgroups per compute unit.
-// Measured, four waves and sixteen: 28 tiles of 93 entries 27 and 20.5 us, 256 tiles of 76 entries 30 and 25.6, of 760
-// 151 and 103, of 560 with large splats 69 and 51, 512 tiles of 440 entries 102 and 76, 512 of 390 and of 2600 with
-// large splats (most behind opaque ones) 69 and 63, 62.8 and 61.7. With T and the back-sum run through all four
-// entries in every group (three exchanges of four values) 256 tiles of 760 took 110 us, 512 of large splats 67 to 69.
-constexpr int kWideSeg = 64;  // a block's entries per segment (41 KB of sums: two workgroups per compute unit)
-
-__global__ void __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) k_raster_bwd_wide(RasterArgs a, const float* __restrict__ ralpha,
-                                                                  const int32_t* __restrict__ last_ids,
-                                                                  const float* __restrict__ v_rc,
-                                                                  const float* __restrict__ v_ra, RasterBwdGrads g) {
-    constexpr int kEntWords = kGrads + 1;
-    constexpr int kPad = kThreads * static_cast<int>(sizeof(float4));  // the record no pixel reaches
-    static_assert(kWideThreads == 64 * kBlocks && kWideThreads == 4 * kThreads, "a wave per block, four threads per slot");
-    // as in k_raster_bwd; batches of kThreads slots, staged by the first four waves
-    __shared__ float4 s_xyo[kThreads + 1];
-    __shared__ float4 s_con[kThreads + 1];
-    __shared__ float4 s_rgb[kThreads + 1];
-    __shared__ __align__(16) float s_ent[kBlocks][kWideSeg][kEntWords];
-    __shared__ unsigned long long s_bits[kBlocks][4];
-    __shared__ __align__(8) uint16_t s_seg[kBlocks][kWideSeg];
-    __shared__ uint8_t s_epos[kThreads][kBlocks];
-    __shared__ uint16_t s_bm[kThreads];
-    __shared__ int32_t s_bbf[kBlocks];
-    __shared__ unsigned long long s_gen[4];
-    const int n_tiles = a.tile_width * a.tile_height;
-    const int img = blockIdx.x / n_tiles;
-    const int tile = a.tile_order ? a.tile_order[blockIdx.x % n_tiles] : static_cast<int>(blockIdx.x % n_tiles);
-    if (a.masks && a.masks[(size_t)img * n_tiles + tile] == 0) return;  // uniform
-    const int tx = tile % a.tile_width, ty = tile / a.tile_width;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, bl = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's block
-    const int grp = lane >> 4, r = lane & 15;
-    const int px_i = tx * 16 + 4 * (bl & 3) + (r & 3), py_i = ty * 16 + 4 * (bl >> 2) + (r >> 2);
-    const bool inside = px_i < a.width && py_i < a.height;
-    const size_t pix = inside ? (size_t)img * a.height * a.width + (size_t)py_i * a.width + px_i
-                              : (size_t)img * a.height * a.width;
-    const int32_t* offs = a.offsets + (size_t)img * n_tiles;
-    const int32_t range_start = offs[tile];
-    const int32_t range_end = (img == a.I - 1 && tile == n_tiles - 1)
-                                  ? (a.n_isects_dev ? static_cast<int32_t>(*a.n_isects_dev) : a.n_isects)
-                                  : offs[tile + 1];
-    const float px = static_cast<float>(px_i) + 0.5f, py = static_cast<float>(py_i) + 0.5f;
-    const float T_final = 1.0f - ralpha[pix];
-    float T = T_final;
-    float bdot = 0.f;
-    const int32_t bin_final = inside ? last_ids[pix] : -1;
-    const float vc0 = v_rc[pix * 3], vc1 = v_rc[pix * 3 + 1], vc2 = v_rc[pix * 3 + 2];
-    float tva;
-    {
-        const float* bg = a.backgrounds ? a.backgrounds + img * 3 : nullptr;
-        const float bg_dot = bg ? (bg[0] * vc0 + bg[1] * vc1 + bg[2] * vc2) : 0.f;
-        tva = T_final * (v_ra[pix] - bg_dot);
-    }
-    {
-        const int32_t block_bin_final = row_max16(bin_final);
-        if (lane == 0) s_bbf[bl] = block_bin_final;
-    }
-    if (tid == 0) {
-        s_xyo[kThreads] = make_float4(0.f, 0.f, 0.f, -__builtin_inff());
-        s_con[kThreads] = make_float4(0.f, 0.f, 0.f, 0.f);
-        s_rgb[kThreads] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    __syncthreads();
-    int32_t tile_bf = s_bbf[0];
-#pragma unroll
-    for (int k = 1; k < kBlocks; k++) tile_bf = max(tile_bf, s_bbf[k]);
-    const int32_t tile_end = min(range_end, __builtin_amdgcn_readfirstlane(tile_bf) + 1);
-    const int32_t num = max(0, tile_end - range_start);
-    const int32_t mask_end = a.block_masks ? a.mask_end[(size_t)img * n_tiles + tile] : range_start;
-    const int num_batches = (num + kThreads - 1) / kThreads;
-    // group_sum4 leaves component 0 (of its four) in lane 0 of the group, 1 in 8, 2 in 4, 3 in 12
-    const bool writes = (r & 3) == 0;
-    const int comp = ((r >> 3) & 1) | ((r >> 1) & 2);
-    for (int b = 0; b < num_batches; b++) {
-        __syncthreads();  // the previous batch's flush has read the records
-        const int32_t batch_end = tile_end - 1 - kThreads * b;
-        const int32_t batch_size = min(kThreads, batch_end + 1 - range_start);
-        if (tid < kThreads) {
-            const int32_t idx = batch_end - tid;
-            uint32_t bm = 0u;
-            bool big = false;
-            if (idx >= range_start) {
-                const int32_t f = a.flatten_ids[idx];
-                const int32_t gid = a.id_of ? a.id_of[f] : f;
-                float4 xyo = a.splats[(size_t)gid * 3];
-                xyo.w = sigma_cutoff(xyo.z);
-                float4 con = a.splats[(size_t)gid * 3 + 1];
-                float4 rgb = a.splats[(size_t)gid * 3 + 2];
-                bm = idx < mask_end ? static_cast<uint32_t>(a.block_masks[idx])
-                                    : block_mask(xyo, con, static_cast<float>(tx * 16), static_cast<float>(ty * 16));
-#pragma unroll
-                for (int k = 0; k < kBlocks; k++)
-                    if (idx > s_bbf[k]) bm &= ~(1u << k);
-                big = bm != 0u && xyo.w > 86.0f;
-                xyo.w -= kCutoffMargin;
-                con.w = __int_as_float(gid);
-                rgb.w = __int_as_float(f);
-                s_xyo[tid] = xyo;
-                s_con[tid] = con;
-                s_rgb[tid] = rgb;
-            }
-            s_bm[tid] = static_cast<uint16_t>(bm);
-#pragma unroll
-            for (int k = 0; k < kBlocks; k++) {
-                const unsigned long long bal = __ballot((bm >> k) & 1u);
-                if (lane == 0) s_bits[k][bl] = bal;
-            }
-            const unsigned long long gb = __ballot(big);
-            if (lane == 0) s_gen[bl] = gb;
-        }
-        __syncthreads();
-        const bool general = (s_gen[0] | s_gen[1] | s_gen[2] | s_gen[3]) != 0ull;
-        const int tmin16 = (batch_end - bin_final) * static_cast<int>(sizeof(float4));
-        for (int s0 = 0; s0 < batch_size;) {  // uniform: every wave derives the same bounds
-            const int lim = row_min16(seg_limit(s_bits[lane & (kBlocks - 1)], s0, kWideSeg));
-            const int s1 = max(s0 + 1, min(static_cast<int>(batch_size), __builtin_amdgcn_readfirstlane(lim)));
-            // the block's list of the segment: lane l takes slots l, 64 + l, ... (at most kWideSeg are set)
-            int cnt = 0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int lo = min(max(s0 - 64 * i, 0), 64), hi = min(max(s1 - 64 * i, 0), 64);
-                const unsigned long long mhi = hi >= 64 ? ~0ull : ((1ull << hi) - 1ull);
-                const unsigned long long mlo = lo >= 64 ? ~0ull : ((1ull << lo) - 1ull);
-                const unsigned long long w = s_bits[bl][i] & mhi & ~mlo;
-                const int pos = cnt + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(w >> 32),
-                                                                                __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(w), 0u)));
-                if (((w >> lane) & 1ull) && pos < kWideSeg) {
-                    const int slot = 64 * i + lane;
-                    s_seg[bl][pos] = static_cast<uint16_t>(slot * sizeof(float4));
-                    s_epos[slot][bl] = static_cast<uint8_t>(pos);
-                }
-                cnt += __popcll(w);
-            }
-            cnt = __builtin_amdgcn_readfirstlane(cnt);
-            if (lane < 4 && cnt + lane < kWideSeg) s_seg[bl][cnt + lane] = static_cast<uint16_t>(kPad);
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // lanes read what others wrote
-            const char* const lds_xyo = reinterpret_cast<const char*>(s_xyo);
-            const char* const lds_con = reinterpret_cast<const char*>(s_con);
-            const char* const lds_rgb = reinterpret_cast<const char*>(s_rgb);
-            auto walk = [&](auto gen_batch) {
-                int next = s_seg[bl][grp];
-                for (int j = 0; j < cnt; j += 4) {  // (positions past the list: the pad, or sums that nothing reads)
-                    const int off = next;
-                    next = s_seg[bl][min(j + 4, kWideSeg - 4) + grp];
-                    const float4 xyo = *reinterpret_cast<const float4*>(lds_xyo + off);
-                    const float4 con = *reinterpret_cast<const float4*>(lds_con + off);
-                    const float dx = xyo.x - px, dy = xyo.y - py;
-                    const float sig = sigma_of(con.x, con.y, con.z, dx, dy);
-                    const bool valid = (off >= tmin16) & !(sig - xyo.w > kCutoffMargin) & !(sig < 0.f);
-                    float* const ent = s_ent[bl][j + grp];
-                    if (!__any(valid)) {  // uniform: T, the back-sum and the gradients unchanged
-                        if (writes) {
-                            ent[comp] = 0.f;
-                            ent[4 + comp] = 0.f;
-                            if (r == 0) ent[8] = 0.f;
-                        }
-                        continue;
-                    }
-                    const float4 rgb = *reinterpret_cast<const float4*>(lds_rgb + off);
-                    const float e = decltype(gen_batch)::value ? sxm::expf_fast(-sig) : exp_neg_poly(sig);
-                    const float oa = xyo.z * e;
-                    const float alpha_raw = sxd::smin(sx::kMaxAlpha, oa);
-                    const bool ok = valid & !(alpha_raw < sx::kAlphaThreshold);
-                    const float alpha = ok ? alpha_raw : 0.0f;
-                    const float vis = (ok & (oa <= sx::kMaxAlpha)) ? e : 0.0f;
-                    const float ra = __builtin_amdgcn_rcpf(1.0f - alpha);
-                    const float cvc = __builtin_fmaf(rgb.x, vc0, __builtin_fmaf(rgb.y, vc1, rgb.z * vc2));
-                    // T through the own entry and the back-sum before it: prefixes over the four groups
-                    const auto pr = pair_of(ra);
-                    const float r2 = pr.lo * pr.hi;
-                    const auto qr = half_of(r2);
-                    const float pre = (grp & 1) ? r2 : ra;
-                    const float own_T = T * (grp >= 2 ? qr.lo * pre : pre);
-                    T *= qr.lo * qr.hi;
-                    const float fac = alpha * own_T;
-                    const float back = fac * cvc;
-                    const auto pb = pair_of(back);
-                    const float b2 = pb.lo + pb.hi;
-                    const auto qb = half_of(b2);
-                    const float before = (grp & 1) ? pb.lo : 0.f;
-                    const float own_b = bdot + (grp >= 2 ? qb.lo + before : before);
-                    bdot += qb.lo + qb.hi;
-                    const float v_alpha = __builtin_fmaf(own_T, cvc, ra * (tva - own_b));
-                    const float gw = vis * v_alpha;
-                    const float wdx = gw * dx, wdy = gw * dy;
-                    const float u0 = group_sum4(wdx, wdy, gw, wdx * dx);
-                    const float u1 = group_sum4(wdx * dy, wdy * dy, fac * vc0, fac * vc1);
-                    const float c2 = fac * vc2;
-                    float u2 = c2 + dpp_f<0x128>(c2);  // group_sum4's order: row_ror:8, row_half_mirror, the quads
-                    u2 += dpp_f<0x141>(u2);
-                    u2 += dpp_f<0xB1>(u2);
-                    u2 += dpp_f<0x4E>(u2);
-                    if (writes) {
-                        ent[comp] = u0;
-                        ent[4 + comp] = u1;
-                        if (r == 0) ent[8] = u2;
-                    }
-                }
-            };
-            if (general)  // uniform
-                walk(std::true_type{});
-            else
-                walk(std::false_type{});
-            __syncthreads();
-            // the segment's totals: four threads a slot, thread q the components 2q and 2q + 1 (the last also 8), each
-            // over the blocks the slot reaches in their order
-            const int slot = s0 + (tid >> 2), part = tid & 3;
-            uint32_t m = slot < s1 ? static_cast<uint32_t>(s_bm[slot]) : 0u;
-            if (m) {
-                float v0 = 0.f, v1 = 0.f, v8 = 0.f;
-                while (m) {
-                    const int b2 = __builtin_ctz(m);
-                    m &= m - 1u;
-                    const float* ent = s_ent[b2][s_epos[slot][b2]];
-                    const float2 x = *reinterpret_cast<const float2*>(ent + 2 * part);
-                    v0 += x.x;
-                    v1 += x.y;
-                    v8 += ent[8];
-                }
-                const float4 cn = s_con[slot];
-                const float nop = -s_xyo[slot].z;
-                if (part == 0) {
-                    const float sdx = v0, sdy = v1;
-                    v0 = __builtin_fmaf(cn.x, sdx, cn.y * sdy) * nop;
-                    v1 = __builtin_fmaf(cn.y, sdx, cn.z * sdy) * nop;
-                } else if (part == 1) {
-                    v1 *= 0.5f * nop;
-                } else if (part == 2) {
-                    v0 *= nop;
-                    v1 *= 0.5f * nop;
-                }
-                const int32_t f = __float_as_int(s_rgb[slot].w);
-                if (g.part) {
-                    float* dst = g.part + (size_t)f * kPartStride;
-                    *reinterpret_cast<float2*>(dst + 2 * part) = make_float2(v0, v1);
-                    if (part == 3) *reinterpret_cast<float4*>(dst + 8) = make_float4(v8, __uint_as_float(*g.stamp), 0.f, 0.f);
-                    if (part == 0) g.touched[__float_as_int(cn.w)] = 1;
-                } else {
-                    if (v0 != 0.f) atomicAdd(grad_slot(g, f, 2 * part), v0);
-                    if (v1 != 0.f) atomicAdd(grad_slot(g, f, 2 * part + 1), v1);
-                    if (part == 3 && v8 != 0.f) atomicAdd(grad_slot(g, f, 8), v8);
-                }
-            }
-            __syncthreads();  // the next segment overwrites the entries and the lists
-            s0 = s1;
-        }
-    }
-}
-
 } // namespace
 
 namespace {
@@ -1625,8 +1355,6 @@ void raster_bwd(const RasterArgs& a, const float* ralpha, const int32_t* last_id
     else if (a.stats)
         hipLaunchKernelGGL((k_raster_bwd<false, true, kBwdSeg>), dim3(blocks), dim3(kThreads), 0, s, a, ralpha, last_ids,
                            v_rc, v_ra, g);
-    else if (blocks <= kWideTiles)
-        hipLaunchKernelGGL(k_raster_bwd_wide, dim3(blocks), dim3(kWideThreads), 0, s, a, ralpha, last_ids, v_rc, v_ra, g);
     else
         hipLaunchKernelGGL((k_raster_bwd<false, false, kBwdSeg>), dim3(blocks), dim3(kThreads), 0, s, a, ralpha, last_ids,
                            v_rc, v_ra, g);

@@ -1,6 +1,7 @@
-"""The rasterisers on images of few tiles (a wave per 4x4 pixel block) and around the tile count where they change to
-four waves a tile (512): lists around the batch (512 entries) and chunk (4) edges, where a pixel's transmittance is
-spent within a chunk, colours that a zero weight would not cancel, masks, backgrounds and several images."""
+"""The rasterisers on images of few tiles (the forward has a wave per 4x4 pixel block there) and around the tile count
+where it changes to four waves a tile (512): lists around the batch (512 entries) and chunk (4) edges, where a pixel's
+transmittance is spent within a chunk, colours that a zero weight would not cancel, masks, backgrounds and several
+images."""
 import numpy as np
 import pytest
 
@@ -48,8 +49,8 @@ def test_spent_within_a_chunk(gpu, oracle, opacity):
 
 @pytest.mark.parametrize("n", [63, 64, 65, 127, 129, 255, 256, 257, 321])
 def test_backward_segments(gpu, oracle, n):
-    """Faint splats over every pixel: each block's list holds all entries, around the segment (64) and the batch (256)
-    of the backward. The sums run over 16 pixels and 16 blocks in 32 bits, T over n factors: below 1e-4."""
+    """Faint splats over every pixel: each block's list holds all entries, around two segments (32 each) and
+    the batch (256) of the backward. The sums run over 16 pixels and 16 blocks in 32 bits, T over n factors: below 1e-4."""
     kw = extreme_splats(20 + n, n=n, width=33, height=18)
     kw["opacities"] = np.full_like(kw["opacities"], 0.02)
     kw["conics"] = np.tile(np.array([0.002, 0.0005, 0.003], np.float32), (1, n, 1))
@@ -71,3 +72,39 @@ def test_colours_not_finite(gpu, oracle):
 
 def test_images_masks_backgrounds(gpu, oracle):
     check(gpu, oracle, inputs.raster_kwargs(oracle, n=900, seed=11, I=2, width=75, height=45, backgrounds=True, masks=True))
+
+
+@pytest.mark.parametrize("n", [1, 3, 5, 63, 65, 300, 1000])
+def test_same_bits_among_many_images(gpu, n):
+    """One image of six tiles, and the same image 100 times in one call (600 tiles): the forward and the gradients of an
+    image do not depend on the tiles beside it, bit for bit. Each tile lists splats of its own, so that every gradient
+    is one sum of one tile and no order of atomic adds enters."""
+    print(f"entries {n}", flush=True)
+    many, w, h, tiles = 100, 44, 29, 6
+    one = extreme_splats(70 + n, n=tiles * n, width=w, height=h)
+    one["flatten_ids"] = np.arange(tiles * n, dtype=np.int32)
+    one["isect_offsets"] = (np.arange(tiles, dtype=np.int32) * n).reshape(1, 2, 3)
+    one["n_isects"] = tiles * n
+    all_ = dict(one, I=many, n_isects=many * tiles * n)
+    for k in ("means2d", "conics", "colors", "opacities"):
+        all_[k] = np.repeat(one[k], many, 0)
+    for k in ("flatten_ids", "isect_offsets"):
+        step = np.arange(many, dtype=np.int32) * (tiles * n)
+        all_[k] = (one[k].reshape(1, -1) + step[:, None]).astype(np.int32)
+    all_["flatten_ids"] = all_["flatten_ids"].ravel()
+    all_["isect_offsets"] = all_["isect_offsets"].reshape(many, 2, 3)
+    a, b = gpu.rasterize_fwd(**one), gpu.rasterize_fwd(**all_)
+    r = inputs.rng(5)
+    v_c = r.standard_normal(a["render_colors"].shape).astype(np.float32)
+    v_a = r.standard_normal(a["render_alphas"].shape).astype(np.float32)
+    ga = gpu.rasterize_bwd(a["render_alphas"], a["last_ids"], v_c, v_a, **one)
+    gb = gpu.rasterize_bwd(b["render_alphas"], b["last_ids"], np.repeat(v_c, many, 0), np.repeat(v_a, many, 0), **all_)
+    assert np.abs(ga["v_means2d"]).max() > 0
+    for k in range(many):
+        assert same_bits(a["render_colors"][0], b["render_colors"][k]) and same_bits(a["render_alphas"][0], b["render_alphas"][k])
+        # (positions in the list, from the image's first; a pixel no splat reached reads 0 in every image)
+        assert np.array_equal(np.where(a["render_alphas"][0, ..., 0] > 0, a["last_ids"][0] + k * tiles * n, 0), b["last_ids"][k])
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        x = gb[k].reshape(many, *ga[k].shape)
+        for q in range(many):
+            assert same_bits(ga[k], x[q]), (k, q)
