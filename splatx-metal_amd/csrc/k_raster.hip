@@ -803,8 +803,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
 
         const int t_min = batch_end - bin_final;  // slots t >= t_min are at or before the lane's last contributor
         // the same bound on the list's record offsets (slot * 16; the padding record at kThreads * 16 passes
-        // it whenever any slot does, and fails the cutoff)
-        const int tmin16 = t_min * static_cast<int>(sizeof(float4));
+        // it whenever any slot does, and fails the cutoff). Held to the slots' range first: a pixel outside the
+        // image (bin_final -1) in a list past index 2^27 would otherwise wrap around and pass every slot.
+        const int tmin16 = min(max(t_min, 0), kThreads + 1) * static_cast<int>(sizeof(float4));
         // The batch's slots are walked in segments [s0, s1), each ending before the slot of the entry
         // with which some block's list would pass kSeg entries; so the lists are as long as the entry
         // buffer allows whatever the slots' density (fixed 32-slot segments left ~6 entries per list,

@@ -108,3 +108,26 @@ def test_same_bits_among_many_images(gpu, n):
         x = gb[k].reshape(many, *ga[k].shape)
         for q in range(many):
             assert same_bits(ga[k], x[q]), (k, q)
+
+
+def test_backward_far_into_the_list(gpu):
+    """A tile whose list begins past entry 2^27 of the intersections (the entries before it belong to a masked tile, which
+    is skipped): the same gradients, bit for bit, as with the list at the start. The image cuts through its 4x4 blocks,
+    whose pixels outside must take no part."""
+    n, far, w, h = 300, (1 << 27) + 5, 18, 11
+    kw = extreme_splats(12, n=n, width=w, height=h)
+    kw.update(masks=np.array([[[0, 1]]], np.uint8), isect_offsets=np.zeros((1, 1, 2), np.int32),
+              flatten_ids=np.arange(n, dtype=np.int32), n_isects=n)
+    ids = np.zeros(far + n, np.int32)
+    ids[far:] = kw["flatten_ids"]
+    moved = dict(kw, isect_offsets=np.array([[[0, far]]], np.int32), flatten_ids=ids, n_isects=far + n)
+    r = inputs.rng(5)
+    v_c, v_a = r.standard_normal((1, h, w, 3)).astype(np.float32), r.standard_normal((1, h, w, 1)).astype(np.float32)
+    g = []
+    for k in (kw, moved):
+        f = gpu.rasterize_fwd(**k)
+        g.append((f, gpu.rasterize_bwd(f["render_alphas"], f["last_ids"], v_c, v_a, **k)))
+    assert same_bits(g[0][0]["render_colors"], g[1][0]["render_colors"])
+    assert np.abs(g[0][1]["v_means2d"]).max() > 0
+    for k in ("v_means2d", "v_conics", "v_colors", "v_opacities"):
+        assert same_bits(g[0][1][k], g[1][1][k]), k
