@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(kThreads) k_rs_count(const K* __restrict__ key
     __syncthreads();
     const int64_t i0 = (int64_t)tile * kTile + (int64_t)threadIdx.x * kRounds;
     K key[kRounds];
-    if (i0 + kRounds <= n) {  // the tile is 16-B aligned (4096 keys), and so is each thread's part
+    if (i0 + kRounds <= n) {  // the library's own buffers: a tile (4096 keys) is 16-B aligned, and so is each thread's part
         constexpr int kVec = kRounds * sizeof(K) / 16;
         uint4 w[kVec];
 #pragma unroll
@@ -442,8 +442,11 @@ __global__ void __launch_bounds__(T) k_row_count(const K* __restrict__ keys, int
     __syncthreads();
     const int64_t i0 = (int64_t)tile * (kThreads * R) + (int64_t)threadIdx.x * R;
     K key[R];
-    if (i0 + R <= n) {  // whole vectors: a thread's keys start at a multiple of their size
-        using V = typename std::conditional<R * sizeof(K) % 16 == 0, uint4, uint2>::type;
+    // whole vectors where the array starts at a multiple of a vector (a thread's keys then do too); a caller's own
+    // device buffers (the allocation-free sort) need no more than a key's alignment
+    using V = typename std::conditional<R * sizeof(K) % 16 == 0, uint4, uint2>::type;
+    const bool aligned = (reinterpret_cast<uintptr_t>(keys) & (sizeof(V) - 1)) == 0;  // uniform
+    if (aligned && i0 + R <= n) {
         constexpr int kVec = R * sizeof(K) / sizeof(V);
         static_assert(kVec * sizeof(V) == R * sizeof(K), "a thread's keys are whole vectors");
         V w[kVec];

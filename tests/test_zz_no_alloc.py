@@ -1,8 +1,8 @@
 """sxh_sort_isect_noalloc (the allocation-free device-buffer sort) against sxh_sort_isect.
 
 Two calls in a row on the same device share the library's scratch array: the first at the array's
-capacity (2^21 keys, 45-bit keys: 6 passes, the result's last pass lands in the output after an even
-count), the second smaller (36-bit keys: 5 passes, odd), over what the first left in the array. Each
+capacity (2^21 keys, 45-bit keys: 5 passes, an odd count, after which the last pass lands in the other
+buffer), the second smaller (36-bit keys: 4 passes, even), over what the first left in the array. Each
 result is compared bit for bit with the staged entry point's, whose sort is the same. Then the
 rejections: one key over the capacity, a host pointer, an output aliasing its input (the same address
 or one element past it), outputs overlapping each other, buffers shorter than n elements.
