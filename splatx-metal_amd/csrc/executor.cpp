@@ -118,17 +118,12 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
         for (int g = 0; g < 6; g++)
             if (e->dims[g] > 0 && (!s->params[g] || !s->exp_avg[g] || !s->exp_avg_sq[g]))
                 invalid("TrainStepExecutor", "null parameter/moment pointer for group " + std::to_string(g));
-    if (up && !(e->permuted && rows >= e->perm_count)) {
-        sxh_detail::canonicalize(e);  // rows in the caller's order, the pending update applied
-    } else {
-        // a download puts each row in its caller's place as it packs it, and the arena keeps its order; an
-        // upload over every permuted row replaces them all, so they need not move back first
-        sxh_detail::flush_update(e);
-        if (up) {
-            e->permuted = false;
-            e->steps_since_exchange = 0;
-        }
-    }
+    // a download puts each row in its caller's place as it packs it, and the arena keeps its order; an upload over
+    // every permuted row replaces them all, so they need not move back first
+    const bool over = up && e->permuted && rows >= e->perm_count;
+    if (up && !over) sxh_detail::canonicalize(e);  // rows in the caller's order, the pending update applied
+    else sxh_detail::flush_update(e);
+    if (up) e->steps_since_exchange = 0;
     if (rows == 0) return;
     // rows packed: with the arena in spatial order a row below `rows` may stand anywhere in the permuted part
     const int n_pack = e->permuted ? std::max(rows, e->perm_count) : rows;
@@ -139,6 +134,7 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
     for (int g = 0; g < 6; g++) floats += static_cast<int64_t>(rows) * e->dims[g] * 3;
     const bool one_block = static_cast<size_t>(floats) <= e->staging.n;
     float* at = e->staging.p;
+    bool moved[6][3] = {};  // the arrays whose rows an upload has replaced
     for (int g = 0; g < 6; g++) {
         const int dim = e->dims[g];
         if (dim == 0) continue;
@@ -148,14 +144,36 @@ static void sync_params(sxh_executor* e, const sxh_param_sync* s, bool up) {
             // (side by side where the staging buffer holds all; else one after another in it, in stream order)
             XferItem it{host[k], at, static_cast<size_t>(rows) * dim * 4, {}};
             float* const col = dev[k];
-            if (up) it.stage = [=] { sxk::rows_to_soa(at, col, rows, dim, e->rows, st); };
+            bool* const done = &moved[g][k];
+            if (up) it.stage = [=] {
+                sxk::rows_to_soa(at, col, rows, dim, e->rows, st);
+                *done = true;
+            };
             else it.stage = [=] { sxk::soa_to_rows(col, at, n_pack, dim, e->rows, st, place, e->perm_count, rows); };
             items.push_back(std::move(it));
             if (one_block) at += static_cast<size_t>(rows) * dim;
         }
     }
-    if (up) e->b->xfer->to_device(items, st);
-    else e->b->xfer->to_host(items, st);
+    if (!up) {
+        e->b->xfer->to_host(items, st);
+    } else {
+        try {
+            e->b->xfer->to_device(items, st);
+        } catch (...) {
+            if (over) {  // the arrays the upload did not reach: back to the caller's order, as the others are
+                sxk::Arena left = e->arena();
+                for (int g = 0; g < 6; g++) {
+                    if (moved[g][0]) left.p[g] = nullptr;
+                    if (moved[g][1]) left.m[g] = nullptr;
+                    if (moved[g][2]) left.v[g] = nullptr;
+                }
+                sxk::arena_permute_rows(left, e->dims, e->perm_count, e->row_int.p, e->staging.p, st);
+                e->permuted = false;
+            }
+            throw;
+        }
+        if (over) e->permuted = false;
+    }
     SXH_HIP(hipGetLastError());
     SXH_HIP(hipStreamSynchronize(st));
 }

@@ -235,6 +235,7 @@ void arena_permute_rows(const Arena& A, const int dims[6], int count, const int3
     for (int g = 0; g < 6; g++) {
         if (dims[g] == 0) continue;
         for (float* col : {A.p[g], A.m[g], A.v[g]}) {
+            if (!col) continue;
             soa_to_rows(col, tmp, count, dims[g], A.rows, s);
             rows_to_soa(tmp, col, count, dims[g], A.rows, s, src);
         }

@@ -169,7 +169,7 @@ void step_update_preprocess(const StepConst& cu, const StepConst& c, const Arena
 // The arena's spatial order (row_orig[k]: the original row of internal row k; row_int its inverse;
 // nothing is reordered past the live rows [0, count)). arena_morton_keys: keys[i] = the 30-bit Morton
 // code of row i's mean in the means' bounding box, vals[i] = i (scratch: arena_morton_scratch_floats).
-// arena_permute_rows: internal row k of every parameter and moment column takes row src[k] (tmp:
+// arena_permute_rows: internal row k of every parameter and moment column (null: left out) takes row src[k] (tmp:
 // 45 * count floats at least). perm_maps: the maps of src read as internal row k <- original row src[k].
 void arena_morton_keys(const Arena& A, int count, float* scratch, uint32_t* keys, int32_t* vals, hipStream_t s);
 size_t arena_morton_scratch_floats(int count);

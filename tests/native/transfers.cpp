@@ -1,0 +1,180 @@
+// The executor's exchange of rows, the pinned ring and the device buffers' cache on a runtime of host memory
+// (host_runtime.h). One check per argument; the kernels that move rows are written out here as their headers state them.
+#include <cstdio>
+#include <cstdlib>
+#include <functional>
+#include <map>
+#include <string>
+#include <thread>
+#include <vector>
+
+#include "host_runtime.h"
+#include "sx_exec.h"
+#include "sx_host.h"
+#include "sx_kernels.h"
+#include "sx_step.h"
+
+#define CHECK(x)                                                        \
+    do {                                                                \
+        if (!(x)) {                                                     \
+            std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);         \
+            std::exit(1);                                               \
+        }                                                               \
+    } while (0)
+
+namespace sxh {
+static thread_local std::string g_error;
+void set_last_error(const std::string& m) { g_error = m; }
+}  // namespace sxh
+
+namespace sxk {
+size_t scan_scratch_bytes(int64_t) { return 64; }
+size_t sort_scratch_bytes(int64_t) { return 64; }
+int step_preprocess_blocks(int64_t n) { return static_cast<int>((n + 255) / 256); }
+void copy_bytes(void* dst, const void* src, size_t n, hipStream_t s) {
+    host_runtime::enqueue(s, [=] { std::memcpy(dst, src, n); });
+}
+void soa_to_rows(const float* soa, float* aos, int n, int dim, int stride, hipStream_t s, const int32_t* dst_row, int n_perm,
+                 int n_out) {
+    host_runtime::enqueue(s, [=] {
+        for (int k = 0; k < n; k++) {
+            const int to = dst_row && k < n_perm ? dst_row[k] : k;
+            if (to < (n_out < 0 ? n : n_out))
+                for (int d = 0; d < dim; d++) aos[(size_t)to * dim + d] = soa[(size_t)d * stride + k];
+        }
+    });
+}
+void rows_to_soa(const float* aos, float* soa, int n, int dim, int stride, hipStream_t s, const int32_t* src_row) {
+    host_runtime::enqueue(s, [=] {
+        for (int k = 0; k < n; k++)
+            for (int d = 0; d < dim; d++) soa[(size_t)d * stride + k] = aos[(size_t)(src_row ? src_row[k] : k) * dim + d];
+    });
+}
+void arena_permute_rows(const Arena& A, const int dims[6], int count, const int32_t* src, float* tmp, hipStream_t s) {
+    for (int g = 0; g < 6; g++)
+        for (float* col : {A.p[g], A.m[g], A.v[g]}) {
+            if (!col || dims[g] == 0) continue;
+            soa_to_rows(col, tmp, count, dims[g], A.rows, s);
+            rows_to_soa(tmp, col, count, dims[g], A.rows, s, src);
+        }
+}
+}  // namespace sxk
+
+namespace {
+
+struct Backend {
+    sxh_backend* b = new sxh_backend;
+    Backend() {
+        SXH_HIP(hipStreamCreateWithFlags(&b->stream, 0));
+        b->xfer = std::make_unique<sxh::HostXfer>(0);
+    }
+    ~Backend() {
+        b->xfer.reset();
+        b->cache.release();
+        (void)hipStreamDestroy(b->stream);
+        delete b;
+    }
+};
+
+// Parameters and moments of `rows` rows at SH degree 1, every value its own; array `pin` (of 18) in pinned memory.
+struct Rows {
+    std::vector<float> a[3][6];
+    float* pinned = nullptr;
+    int pin;
+    static constexpr int kDims[6] = {3, 4, 3, 1, 3, 9};
+    Rows(int rows, float first, int pin_at = -1) : pin(pin_at) {
+        for (int g = 0; g < 6; g++)
+            for (int k = 0; k < 3; k++) {
+                a[k][g].resize((size_t)rows * kDims[g]);
+                for (size_t q = 0; q < a[k][g].size(); q++) a[k][g][q] = first + 1000.0f * (3 * g + k) + q * 0.25f;
+                if (3 * g + k == pin) {
+                    SXH_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), a[k][g].size() * 4, 0));
+                    std::memcpy(pinned, a[k][g].data(), a[k][g].size() * 4);
+                }
+            }
+    }
+    ~Rows() {
+        if (pinned) (void)hipHostFree(pinned);
+    }
+    sxh_param_sync sync(int rows) {
+        sxh_param_sync s{};
+        for (int g = 0; g < 6; g++) {
+            s.params[g] = 3 * g == pin ? pinned : a[0][g].data();
+            s.exp_avg[g] = 3 * g + 1 == pin ? pinned : a[1][g].data();
+            s.exp_avg_sq[g] = 3 * g + 2 == pin ? pinned : a[2][g].data();
+        }
+        s.rows = rows;
+        return s;
+    }
+};
+
+// The arena's first n rows as a training step leaves them in spatial order: internal row k holds row n - 1 - k.
+void reverse_order(sxh_executor* e, int n) {
+    e->row_orig.alloc(e->rows);
+    e->row_int.alloc(e->rows);
+    for (int k = 0; k < n; k++) e->row_orig.p[k] = e->row_int.p[k] = n - 1 - k;
+    sxk::arena_permute_rows(e->arena(), e->dims, n, e->row_orig.p, e->staging.p, e->b->stream);
+    SXH_HIP(hipStreamSynchronize(e->b->stream));
+    e->permuted = true;
+    e->perm_count = n;
+}
+
+sxh_executor* executor(sxh_backend* b, int rows) {
+    sxh_exec_desc d{};
+    d.arena_rows = rows;
+    d.sh_degree = 1;
+    d.isect_mode = SXH_ISECT_ACCUTILE;
+    sxh_executor* e = nullptr;
+    CHECK(sxh_exec_create(b, &d, &e) == SXH_OK);
+    return e;
+}
+
+// An upload over every row of an arena in spatial order that fails at its eighth array: the seven before it hold the
+// new rows, the others the old ones, all in the caller's order, and the next exchange sees them so. At 70,000 rows the
+// arrays travel one by one, at 300 in one block up to the failing one.
+void upload_fails_midway() {
+    for (int n : {300, 70000}) {
+        Backend B;
+        sxh_executor* e = executor(B.b, n);
+        Rows old(n, 0.0f), fresh(n, 0.5f, 7), got(n, -1.0f);
+        auto so = old.sync(n), sf = fresh.sync(n), sg = got.sync(n);
+        CHECK(sxh_exec_upload(e, &so) == SXH_OK);
+        // (below 8 MiB only the array in pinned memory goes through a copy of the runtime's; above, every chunk does)
+        const int before = host_runtime::copies();
+        CHECK(sxh_exec_upload(e, &so) == SXH_OK);
+        const int fail = n == 300 ? 1 : (host_runtime::copies() - before) / 2;
+        for (const bool spatial : {true, false}) {
+            if (spatial) reverse_order(e, n);
+            host_runtime::faults.copy = fail;
+            CHECK(sxh_exec_upload(e, &sf) == SXH_ERR_RUNTIME);
+            CHECK(host_runtime::faults.copy == 0);
+            CHECK(sxh_exec_download(e, &sg) == SXH_OK);
+            int news = 0;
+            for (int q = 0; q < 18; q++) {
+                const auto& x = got.a[q % 3][q / 3];
+                const bool is_new = x == fresh.a[q % 3][q / 3], is_old = x == old.a[q % 3][q / 3];
+                CHECK(is_new != is_old);
+                CHECK(!is_new || news == q);  // (the arrays before the failing one)
+                news += is_new;
+            }
+            CHECK(n > 300 ? news > 0 && news < 18 : news == 7);
+            CHECK(sxh_exec_upload(e, &so) == SXH_OK);
+        }
+        sxh_exec_destroy(e);
+    }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::map<std::string, std::function<void()>> all = {
+        {"upload_fails_midway", upload_fails_midway},
+    };
+    for (int k = 1; k < argc; k++) {
+        const auto it = all.find(argv[k]);
+        CHECK(it != all.end());
+        it->second();
+        std::printf("%s: done\n", argv[k]);
+    }
+    return 0;
+}
