@@ -127,6 +127,10 @@ struct HostXfer::Impl {
     explicit Impl(int d) : device(d) {}
 
     void start(size_t total) {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            err = hipSuccess;  // (a transfer that threw may have left one; no job runs between transfers)
+        }
         if (!ring) {
             char* r = nullptr;
             SXH_HIP(hipHostMalloc(reinterpret_cast<void**>(&r), kChunk * kSlots, hipHostMallocMapped));

@@ -62,6 +62,8 @@ void arena_permute_rows(const Arena& A, const int dims[6], int count, const int3
 
 namespace {
 
+using sxh::DevBuf;
+
 struct Backend {
     sxh_backend* b = new sxh_backend;
     Backend() {
@@ -164,11 +166,48 @@ void upload_fails_midway() {
     }
 }
 
+// A transfer in which a wait fails on the way and then a copy: it reports an error, and the next one reports none.
+void error_is_reported_once() {
+    Backend B;
+    const size_t n = size_t{64} << 20;  // 16 chunks of 4 MiB, twice around the ring
+    DevBuf<char> dev(n);
+    std::vector<char> host(n, 1), back(n);
+    B.b->xfer->to_device({{host.data(), dev.p, n, {}}}, B.b->stream);
+    B.b->xfer->to_host({{back.data(), dev.p, n, {}}}, B.b->stream);  // (waits for the upload's copies; only its own follow)
+    host_runtime::faults.event_sync = 1;
+    host_runtime::faults.copy = 15;
+    bool threw = false;
+    try {
+        B.b->xfer->to_host({{back.data(), dev.p, n, {}}}, B.b->stream);
+    } catch (const std::exception&) {
+        threw = true;
+    }
+    CHECK(threw && host_runtime::faults.event_sync == 0 && host_runtime::faults.copy == 0);
+    for (int k = 0; k < 2; k++) {
+        back.assign(n, 0);
+        B.b->xfer->to_host({{back.data(), dev.p, n, {}}}, B.b->stream);
+        CHECK(back == host);
+        host[5 + k] = 3;
+        B.b->xfer->to_device({{host.data(), dev.p, n, {}}}, B.b->stream);
+    }
+    // a wait that fails by itself is reported by its own transfer
+    B.b->xfer->to_host({{back.data(), dev.p, n, {}}}, B.b->stream);
+    host_runtime::faults.event_sync = 3;
+    threw = false;
+    try {
+        B.b->xfer->to_host({{back.data(), dev.p, n, {}}}, B.b->stream);
+    } catch (const std::exception&) {
+        threw = true;
+    }
+    CHECK(threw);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> all = {
         {"upload_fails_midway", upload_fails_midway},
+        {"error_is_reported_once", error_is_reported_once},
     };
     for (int k = 1; k < argc; k++) {
         const auto it = all.find(argv[k]);
