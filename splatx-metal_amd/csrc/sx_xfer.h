@@ -28,7 +28,8 @@ struct XferItem {
 };
 
 // The ring and its threads, made on first use and given back with the object: 32 MiB of pinned memory, at most
-// four threads, which sleep between transfers. One transfer at a time (a lock held for its duration).
+// four threads, which sleep between transfers. Without that memory the runtime copies the arrays. One transfer at a
+// time (a lock held for its duration).
 class HostXfer {
   public:
     explicit HostXfer(int device);

@@ -60,10 +60,10 @@ struct Block {
     std::vector<Chunk> chunks;
 };
 
-std::vector<Block> blocks_of(const std::vector<XferItem>& items, size_t step, bool up) {
+std::vector<Block> blocks_of(const std::vector<XferItem>& items, size_t step, bool up, bool ring) {
     std::vector<Block> out;
     for (size_t k = 0; k < items.size();) {
-        if (items[k].bytes == 0 || known_memory(items[k].host)) {
+        if (!ring || items[k].bytes == 0 || known_memory(items[k].host)) {
             out.push_back({k, k + 1, {}});
             k++;
             continue;
@@ -126,23 +126,28 @@ struct HostXfer::Impl {
 
     explicit Impl(int d) : device(d) {}
 
-    void start(size_t total) {
+    // The ring and its events; false where there is no pinned memory for it (asked for again with the next transfer).
+    bool make_ring() {
+        char* r = nullptr;
+        bool ok = hipHostMalloc(reinterpret_cast<void**>(&r), kChunk * kSlots, hipHostMallocMapped) == hipSuccess;
+        for (auto& e : ev)
+            if (ok && !e) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            if (r) (void)hipHostFree(r);
+            return false;
+        }
+        ring = r;
+        return true;
+    }
+
+    // Before a transfer: whether there is a ring (without one the runtime copies every array).
+    bool start(size_t total) {
         {
             std::lock_guard<std::mutex> g(mu);
             err = hipSuccess;  // (a transfer that threw may have left one; no job runs between transfers)
         }
-        if (!ring) {
-            char* r = nullptr;
-            SXH_HIP(hipHostMalloc(reinterpret_cast<void**>(&r), kChunk * kSlots, hipHostMallocMapped));
-            try {
-                for (auto& e : ev)
-                    if (!e) SXH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            } catch (...) {
-                (void)hipHostFree(r);
-                throw;
-            }
-            ring = r;
-        }
+        if (!ring && !make_ring()) return false;
         threaded = total >= kThreadedBytes;
         if (threaded && threads.empty()) {
             const int n = std::min<int>(kThreads, std::max(1u, std::thread::hardware_concurrency() / 2));
@@ -151,6 +156,7 @@ struct HostXfer::Impl {
             } catch (const std::system_error&) {  // (the calling thread takes jobs as well)
             }
         }
+        return true;
     }
 
     ~Impl() {
@@ -252,8 +258,8 @@ void HostXfer::to_device(const std::vector<XferItem>& items, hipStream_t s) {
     Impl& x = *p_;
     const size_t total = total_bytes(items);
     std::lock_guard<std::mutex> one(x.call);
-    x.start(total);
-    const std::vector<Block> blocks = blocks_of(items, chunk_bytes(total), true);
+    const bool ring = x.start(total);
+    const std::vector<Block> blocks = blocks_of(items, chunk_bytes(total), true, ring);
     std::vector<const Chunk*> order;  // the chunks of every block
     for (const Block& b : blocks)
         for (const Chunk& c : b.chunks) order.push_back(&c);
@@ -299,8 +305,8 @@ void HostXfer::to_host(const std::vector<XferItem>& items, hipStream_t s) {
     Impl& x = *p_;
     const size_t total = total_bytes(items);
     std::lock_guard<std::mutex> one(x.call);
-    x.start(total);
-    const std::vector<Block> blocks = blocks_of(items, chunk_bytes(total), false);
+    const bool ring = x.start(total);
+    const std::vector<Block> blocks = blocks_of(items, chunk_bytes(total), false, ring);
     try {
         for (const Block& b : blocks) {
             for (size_t k = b.first; k < b.last; k++)

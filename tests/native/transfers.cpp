@@ -202,12 +202,33 @@ void error_is_reported_once() {
     CHECK(threw);
 }
 
+// Where there is no pinned memory for the ring the runtime copies the arrays; once there is, the ring does.
+void without_the_ring() {
+    for (int n : {300, 70000}) {
+        Backend B;
+        sxh_executor* e = executor(B.b, n);
+        for (const bool none : {true, false}) {
+            host_runtime::faults.pinned = none;
+            Rows up(n, none ? 0.0f : 0.5f), got(n, -1.0f);
+            auto su = up.sync(n), sg = got.sync(n);
+            const int before = host_runtime::copies();
+            CHECK(sxh_exec_upload(e, &su) == SXH_OK);
+            CHECK(sxh_exec_download(e, &sg) == SXH_OK);
+            CHECK(!none || host_runtime::copies() - before == 36);
+            for (int k = 0; k < 3; k++)
+                for (int g = 0; g < 6; g++) CHECK(got.a[k][g] == up.a[k][g]);
+        }
+        sxh_exec_destroy(e);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> all = {
         {"upload_fails_midway", upload_fails_midway},
         {"error_is_reported_once", error_is_reported_once},
+        {"without_the_ring", without_the_ring},
     };
     for (int k = 1; k < argc; k++) {
         const auto it = all.find(argv[k]);
