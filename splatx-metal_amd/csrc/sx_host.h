@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <map>
@@ -63,14 +64,32 @@ int32_t guarded(F&& f) {
 }
 
 // Device memory that the per-op entry points used before, kept for their next calls: at most kMost bytes, given
-// back with the backend. The entry points run on the backend's one stream, so a block is used again in stream
-// order. (hipMalloc and hipFree take 10-100 us each, and an entry point has up to twelve buffers.)
+// back with the backend, and before any allocation of the library fails for want of memory (device_alloc). The entry
+// points run on the backend's one stream, so a block is used again in stream order. (hipMalloc and hipFree take 10-100 us
+// each, and an entry point has up to twelve buffers.)
 class DevCache {
   public:
-    DevCache() = default;
+    DevCache() {
+        Registry& r = registry();
+        std::lock_guard<std::mutex> g(r.mu);
+        r.all.push_back(this);
+    }
     DevCache(const DevCache&) = delete;
     DevCache& operator=(const DevCache&) = delete;
-    ~DevCache() { release(); }
+    ~DevCache() {
+        {
+            Registry& r = registry();
+            std::lock_guard<std::mutex> g(r.mu);
+            r.all.erase(std::find(r.all.begin(), r.all.end(), this));
+        }
+        release();
+    }
+    // What every cache of the process holds, back to the devices.
+    static void release_all() {
+        Registry& r = registry();
+        std::lock_guard<std::mutex> g(r.mu);
+        for (DevCache* c : r.all) c->release();
+    }
     void* get(size_t bytes, size_t* got) {
         {
             std::lock_guard<std::mutex> g(mu_);
@@ -83,14 +102,13 @@ class DevCache {
                 return p;
             }
         }
-        // (rounded up, so that calls of about the same size share blocks)
-        *got = (bytes + bytes / 8 + 4095) & ~size_t{4095};
+        // (rounded up, so that calls of about the same size share blocks, unless it is too large to be kept or to be had)
         void* p = nullptr;
-        if (hipMalloc(&p, *got) == hipSuccess) return p;
+        *got = (bytes + bytes / 8 + 4095) & ~size_t{4095};
+        if (*got <= kMost && hipMalloc(&p, *got) == hipSuccess) return p;
         (void)hipGetLastError();
-        release();
-        SXH_HIP(hipMalloc(&p, *got));
-        return p;
+        *got = bytes;
+        return device_alloc(bytes);
     }
     void put(void* p, size_t bytes) {
         {
@@ -109,8 +127,25 @@ class DevCache {
         free_.clear();
         held_ = 0;
     }
+    // Device memory; if there is not enough, once more without what the caches hold.
+    static void* device_alloc(size_t bytes) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        release_all();
+        SXH_HIP(hipMalloc(&p, bytes));
+        return p;
+    }
 
   private:
+    struct Registry {
+        std::mutex mu;
+        std::vector<DevCache*> all;
+    };
+    static Registry& registry() {
+        static Registry* const r = new Registry;  // (never destroyed: a backend may be destroyed at the process's end)
+        return *r;
+    }
     static constexpr size_t kMost = size_t{256} << 20;
     std::mutex mu_;
     std::multimap<size_t, void*> free_;
@@ -143,7 +178,7 @@ struct DevBuf {
         if (!count) return;
         const size_t bytes = std::max<size_t>(count * sizeof(T), 16);
         if (home) p = static_cast<T*>(home->get(bytes, &home_bytes));
-        else SXH_HIP(hipMalloc(reinterpret_cast<void**>(&p), bytes));
+        else p = static_cast<T*>(DevCache::device_alloc(bytes));
         n = count;
     }
     void ensure(size_t count) {

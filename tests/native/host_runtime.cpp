@@ -59,7 +59,7 @@ namespace {
 std::mutex mu;
 std::map<char*, size_t> device, pinned;
 size_t used = 0;
-std::atomic<int> n_copies{0}, delay{0};
+std::atomic<int> n_copies{0}, n_mallocs{0}, delay{0};
 bool fails(int& n) {
     std::lock_guard<std::mutex> g(mu);
     return n > 0 && --n == 0;
@@ -75,6 +75,7 @@ size_t device_bytes() {
     return used;
 }
 int copies() { return n_copies; }
+int mallocs() { return n_mallocs; }
 void stream_delay_us(int us) { delay = us; }
 }  // namespace host_runtime
 using namespace host_runtime;
@@ -102,6 +103,7 @@ hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipMalloc(void** p, size_t n) {
     std::lock_guard<std::mutex> g(mu);
+    n_mallocs++;
     if (used + n > device_limit) return hipErrorOutOfMemory;
     *p = std::malloc(n);
     std::memset(*p, 0xA5, n);

@@ -19,6 +19,6 @@ struct Faults {
 extern Faults faults;
 extern size_t device_limit;   // bytes that hipMalloc hands out in all
 size_t device_bytes();        // bytes in use
-int copies();                 // hipMemcpyAsync calls so far
+int copies(), mallocs();      // hipMemcpyAsync and hipMalloc calls so far
 void stream_delay_us(int us);  // before each thing a stream runs
 }  // namespace host_runtime

@@ -222,6 +222,34 @@ void without_the_ring() {
     }
 }
 
+// What the per-op calls left in a backend's cache is given back before an allocation fails: the executors' (uncached),
+// another backend's, and a cached one that is only to be had without rounding.
+void kept_memory_gives_way() {
+    constexpr size_t kMiB = size_t{1} << 20;
+    Backend A, B;
+    host_runtime::device_limit = 200 * kMiB;
+    { DevBuf<char> x(50 * kMiB, &A.b->cache), y(40 * kMiB, &B.b->cache); }
+    CHECK(host_runtime::device_bytes() > 90 * kMiB);
+    {
+        DevBuf<char> arena(150 * kMiB);
+        CHECK(arena.p && host_runtime::device_bytes() < 151 * kMiB);
+    }
+    { DevBuf<char> x(60 * kMiB, &A.b->cache); }
+    {
+        DevBuf<char> other(190 * kMiB, &B.b->cache);  // (with an eighth more it would pass the limit)
+        CHECK(other.p);
+    }
+    bool threw = false;
+    try {
+        DevBuf<char> most(201 * kMiB);
+    } catch (const std::exception&) {
+        threw = true;
+    }
+    CHECK(threw);
+    { DevBuf<char> x(8, &A.b->cache), y(8, &A.b->cache); }
+    host_runtime::device_limit = ~size_t{0};
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -229,6 +257,7 @@ int main(int argc, char** argv) {
         {"upload_fails_midway", upload_fails_midway},
         {"error_is_reported_once", error_is_reported_once},
         {"without_the_ring", without_the_ring},
+        {"kept_memory_gives_way", kept_memory_gives_way},
     };
     for (int k = 1; k < argc; k++) {
         const auto it = all.find(argv[k]);

@@ -26,7 +26,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["upload_fails_midway", "error_is_reported_once", "without_the_ring"])
+@pytest.mark.parametrize("check", ["upload_fails_midway", "error_is_reported_once", "without_the_ring", "kept_memory_gives_way"])
 def test_transfers(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
