@@ -95,7 +95,7 @@ class DevCache {
             std::lock_guard<std::mutex> g(mu_);
             const auto it = free_.lower_bound(bytes);
             if (it != free_.end() && it->first <= 2 * bytes + 4096) {
-                void* p = it->second;
+                void* p = it->second.p;
                 *got = it->first;
                 held_ -= it->first;
                 free_.erase(it);
@@ -110,20 +110,31 @@ class DevCache {
         *got = bytes;
         return device_alloc(bytes);
     }
+    // Over kMost, the blocks put back longest ago go, so that what an early burst left does not keep later sizes out.
     void put(void* p, size_t bytes) {
+        std::vector<void*> gone;
         {
             std::lock_guard<std::mutex> g(mu_);
-            if (held_ + bytes <= kMost) {
-                free_.emplace(bytes, p);
+            if (bytes > kMost) {
+                gone.push_back(p);
+            } else {
+                while (held_ + bytes > kMost) {
+                    auto oldest = free_.begin();
+                    for (auto it = free_.begin(); it != free_.end(); ++it)
+                        if (it->second.put < oldest->second.put) oldest = it;
+                    gone.push_back(oldest->second.p);
+                    held_ -= oldest->first;
+                    free_.erase(oldest);
+                }
+                free_.emplace(bytes, Block{p, n_put_++});
                 held_ += bytes;
-                return;
             }
         }
-        (void)hipFree(p);
+        for (void* q : gone) (void)hipFree(q);
     }
     void release() {
         std::lock_guard<std::mutex> g(mu_);
-        for (const auto& f : free_) (void)hipFree(f.second);
+        for (const auto& f : free_) (void)hipFree(f.second.p);
         free_.clear();
         held_ = 0;
     }
@@ -146,10 +157,15 @@ class DevCache {
         static Registry* const r = new Registry;  // (never destroyed: a backend may be destroyed at the process's end)
         return *r;
     }
+    struct Block {
+        void* p;
+        unsigned long long put;  // when it was put back
+    };
     static constexpr size_t kMost = size_t{256} << 20;
     std::mutex mu_;
-    std::multimap<size_t, void*> free_;
+    std::multimap<size_t, Block> free_;  // by size
     size_t held_ = 0;
+    unsigned long long n_put_ = 0;
 };
 
 // Owning device allocation; with a cache, its memory comes from there and goes back there.

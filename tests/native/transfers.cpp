@@ -63,6 +63,7 @@ void arena_permute_rows(const Arena& A, const int dims[6], int count, const int3
 namespace {
 
 using sxh::DevBuf;
+using sxh::DevCache;
 
 struct Backend {
     sxh_backend* b = new sxh_backend;
@@ -250,6 +251,28 @@ void kept_memory_gives_way() {
     host_runtime::device_limit = ~size_t{0};
 }
 
+// After a burst of large sizes has filled the cache, the sizes of later calls are kept all the same, and no more than
+// 256 MiB are.
+void kept_memory_follows_use() {
+    constexpr size_t kMiB = size_t{1} << 20;
+    Backend B;
+    const size_t before = host_runtime::device_bytes();
+    { DevBuf<char> a(70 * kMiB, &B.b->cache), b(75 * kMiB, &B.b->cache), c(80 * kMiB, &B.b->cache); }
+    for (int k = 0; k < 4; k++) {
+        const int n = host_runtime::mallocs();
+        { DevBuf<char> x(20 * kMiB, &B.b->cache), y(3 * kMiB, &B.b->cache), z(100, &B.b->cache); }
+        CHECK(k == 0 || host_runtime::mallocs() == n);
+        CHECK(host_runtime::device_bytes() - before <= 256 * kMiB);
+    }
+    { DevBuf<char> large(300 * kMiB, &B.b->cache); }  // larger than the cache: not kept, and nothing goes for it
+    const int n = host_runtime::mallocs();
+    { DevBuf<char> x(20 * kMiB, &B.b->cache); }
+    CHECK(host_runtime::mallocs() == n);
+    CHECK(host_runtime::device_bytes() - before <= 256 * kMiB);
+    DevCache::release_all();
+    CHECK(host_runtime::device_bytes() == before);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -258,6 +281,7 @@ int main(int argc, char** argv) {
         {"error_is_reported_once", error_is_reported_once},
         {"without_the_ring", without_the_ring},
         {"kept_memory_gives_way", kept_memory_gives_way},
+        {"kept_memory_follows_use", kept_memory_follows_use},
     };
     for (int k = 1; k < argc; k++) {
         const auto it = all.find(argv[k]);
