@@ -507,6 +507,8 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
         uint32_t* const edepth_b =
             index_first ? reinterpret_cast<uint32_t*>(e->keys_a.p) + e->isect_cap : nullptr;
         int which = 0;
+        // (an image of one tile has no tile bits: one pass all the same, which leaves each entry's position as its value)
+        const uint32_t sort_bits = std::max<uint32_t>(1u, c.tile_n_bits);
         // (up to 256 tiles the sort leaves the offsets; the emit clears the words the sort adds into)
         sxk::SortExtra extra{e->offsets.p, n_tiles, false, false};
         sxk::EmitZero zero;
@@ -525,7 +527,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                 sxk::step_emit_sorted(c, e->splats.p, e->radii.p, order, e->cum.p, n_emit, ka, e->emit_gid.p, s,
                                       edepth, zero);
             e->mark("emit");
-            which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
+            which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, sort_bits,
                                               e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &extra);
             e->mark("sort");
             if (!extra.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);
@@ -539,7 +541,7 @@ void sxh_detail::run_step(sxh_executor* e, const sxh_step_inputs* in, sxh_step_o
                 sxk::step_emit_sorted(c, e->splats.p, e->radii.p, order, e->cum.p, n_emit, ka, e->emit_gid.p, s,
                                       edepth, zero);
             e->mark("emit");
-            which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, c.tile_n_bits,
+            which = sxk::radix_sort_positions(ka, e->vals_a.p, kb, e->vals_b.p, n_host, sort_bits,
                                               e->sort_scratch.p, s, index_first, n_dev, edepth, edepth_b, &extra);
             e->mark("sort");
             if (!extra.written) sxk::step_tile_offsets(which ? kb : ka, n_host, n_tiles, e->offsets.p, s, n_dev);

@@ -155,3 +155,30 @@ def test_large_splats_forward_matches_oracle(gpu, isect):
     assert r["n_isects"] == ro["n_isects"] > 100 * sc.n
     assert np.array_equal(r["render_colors"].view(np.uint32), ro["render_colors"].view(np.uint32))
     ex.close()
+
+
+@pytest.mark.parametrize("order", [sh.SXH_ISECT_ORDER_INDEX_FIRST, sh.SXH_ISECT_ORDER_DEPTH_FIRST])
+@pytest.mark.parametrize("n,w,h,ssim", [(1, 16, 16, 0.0), (700, 5, 7, 0.0), (700, 16, 16, 0.2), (5000, 13, 11, 0.2)])
+def test_image_of_one_tile(gpu, n, w, h, ssim, order):
+    """An image within one tile: the tile ids have no bits to sort by, and the list is every row in view by depth. Against
+    the oracle as above."""
+    print(f"rows {n}, {w}x{h}", flush=True)
+    sc = scene.make_scene(n=n, sh_degree=1, width=w, height=h, fx=0.9 * w, seed=19)
+    ex = gpu.make_train_step_executor(arena_rows=n, sh_degree=1, ssim_weight=ssim)
+    ex.set_isect_order(order)
+    g, o = scene.copy_state(sc), scene.copy_state(sc)
+    ex.upload_params(*g, n)
+    kw = scene.step_kwargs(sc)
+    for it in range(3):
+        r = ex.step(want_render=True, gt_rgb=sc.gt, **kw)
+        ro = oracle_py.Oracle(libm=False).train_step(*o, n, 1, sc.viewmat, sc.K, w, h, sc.gt, kw["degrees_to_use"], kw["lr"],
+                                                     ssim_weight=ssim)
+        assert r["n_isects"] == ro["n_isects"] and r["n_visible"] == ro["n_visible"] and (n == 1 or r["n_isects"] > 0)
+        assert abs(r["loss"] - ro["loss"]) <= 1e-6 + 1e-4 * abs(ro["loss"])
+        if it == 0:
+            assert np.array_equal(r["render_colors"].view(np.uint32), ro["render_colors"].view(np.uint32))
+    ex.download_params(*g, n)
+    ex.close()
+    for a, b in zip(g, o):
+        for x, y in zip(a, b):
+            assert rel_l2(x, y) <= 1e-4
