@@ -273,6 +273,35 @@ void kept_memory_follows_use() {
     CHECK(host_runtime::device_bytes() == before);
 }
 
+// Exchanges of many sizes from several threads at once, each thread with a backend of its own, and then all of them on
+// one backend's ring, with streams that lag behind: every thread reads back its own rows.
+void several_threads() {
+    host_runtime::stream_delay_us(30);
+    auto work = [](sxh_backend* b, int seed) {
+        size_t n = 1000 + 4099 * seed;
+        for (int k = 0; k < 12; k++, n = n * 3 + 1) {
+            if (n > size_t{20} << 20) n = 77 + seed;
+            std::vector<char> x(n), y(n), z(n / 2 + 1), w(n / 2 + 1);
+            for (size_t q = 0; q < n; q++) x[q] = static_cast<char>(q * 7 + seed + k);
+            for (size_t q = 0; q < z.size(); q++) z[q] = static_cast<char>(q * 5 - seed);
+            DevBuf<char> d(n, &b->cache), e(z.size(), &b->cache);
+            int staged = 0;
+            b->xfer->to_device({{x.data(), d.p, n, [&] { staged++; }}, {z.data(), e.p, z.size(), [&] { staged++; }}},
+                               b->stream);
+            b->xfer->to_host({{y.data(), d.p, n, [&] { staged++; }}, {w.data(), e.p, w.size(), {}}}, b->stream);
+            CHECK(x == y && z == w && staged == 3);
+        }
+    };
+    std::vector<std::unique_ptr<Backend>> own;
+    for (int k = 0; k < 3; k++) own.push_back(std::make_unique<Backend>());
+    for (const bool one : {false, true}) {
+        std::vector<std::thread> threads;
+        for (int k = 0; k < 3; k++) threads.emplace_back([&, k] { work(own[one ? 0 : k]->b, k); });
+        for (auto& t : threads) t.join();
+    }
+    host_runtime::stream_delay_us(0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -282,6 +311,7 @@ int main(int argc, char** argv) {
         {"without_the_ring", without_the_ring},
         {"kept_memory_gives_way", kept_memory_gives_way},
         {"kept_memory_follows_use", kept_memory_follows_use},
+        {"several_threads", several_threads},
     };
     for (int k = 1; k < argc; k++) {
         const auto it = all.find(argv[k]);

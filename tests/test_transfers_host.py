@@ -27,7 +27,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["upload_fails_midway", "error_is_reported_once", "without_the_ring", "kept_memory_gives_way",
-                                   "kept_memory_follows_use"])
+                                   "kept_memory_follows_use", "several_threads"])
 def test_transfers(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
