@@ -2,6 +2,7 @@
 the sizes where it changes its way (2, 8, 24 and 32 MiB), byte arrays of odd lengths, host memory the runtime already
 knows (pinned), and transfers that follow one another through the same ring."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -36,10 +37,10 @@ def test_byte_masks(gpu, oracle, n):
     assert np.array_equal(got, oracle.sh_fwd(dirs, co, 0, masks=masks))
 
 
-@pytest.mark.parametrize("rows", [70001, 200003])
+@pytest.mark.parametrize("rows", [5001, 30001, 65536, 65537, 70001, 200003])
 def test_large_groups_and_pinned(gpu, rows):
     """Parameters and moments in one exchange, some of them in pinned memory, above and below the size at which the
-    groups are staged together."""
+    groups are staged together (65,536 rows), from a few MB on (copying threads, a copy engine)."""
     hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime the library has loaded
     pinned = []
 
@@ -90,3 +91,37 @@ def test_null_group_is_refused_before_anything_moves(gpu):
     ex.download_params(*got, sc.n)
     ex.close()
     assert all(np.array_equal(x, y) for x, y in zip(got[0], p))
+
+
+def test_backends_on_several_threads():
+    """Backends of their own on three host threads at once: every ring, its threads and its kept buffers are its backend's."""
+    n = 40_003
+    dims = scene.group_dims(2)
+    failed = []
+
+    def work(seed):
+        try:
+            rng = np.random.Generator(np.random.PCG64(seed))
+            b = sh.Backend(0)
+            ex = b.make_train_step_executor(arena_rows=n, sh_degree=2)
+            for k in range(4):
+                up = [[rng.standard_normal((n, d)).astype(np.float32) for d in dims] for _ in range(3)]
+                down = [[np.zeros((n, d), np.float32) for d in dims] for _ in range(3)]
+                ex.upload_params(*up, n)
+                x = rng.integers(0, 100, 300_007 * (seed + k + 1), dtype=np.int32)
+                assert np.array_equal(b.prefix_scan_i64(x), np.cumsum(x, dtype=np.int64))
+                ex.download_params(*down, n)
+                for a, c in zip(up, down):
+                    for y, z in zip(a, c):
+                        assert np.array_equal(y.view(np.uint32), z.view(np.uint32))
+            ex.close()
+            b.close()
+        except Exception as e:  # noqa: BLE001 (told by the test's thread)
+            failed.append((seed, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
