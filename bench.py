@@ -78,8 +78,8 @@ def algorithmic_bytes(name: str, n: int, v: int, i: int, px: int, sh_k: int, sha
         return v * 13.0 + i * 40.0 + v * 48.0
     if name == "depth_sort":
         # compaction: every tile count (4 B) in, the list of Gaussians with tiles (4 B) out; keys: their
-        # depths (4 B) in, (key, index) out (8 B); the onesweep sort of those (u32, i32) pairs: one histogram
-        # read (4 B), per pass a read and a write (16 B)
+        # depths (4 B) in, (key, index) out (8 B); the sort of those (u32, i32) pairs: one read of the keys for the
+        # digit counts (4 B; the later passes' are not counted), per pass a read and a write (16 B)
         return 4.0 * n + v * (4.0 + 4.0 + 8.0) + v * (4.0 + 16.0 * shape["depth_passes"])
     if name == "scan":
         # tile counts gathered through the depth order: order (4 B) + count (4 B) in, offset (8 B) out
@@ -89,8 +89,8 @@ def algorithmic_bytes(name: str, n: int, v: int, i: int, px: int, sh_k: int, sha
         # position's Gaussian) entries out
         return v * (12.0 + 32.0) + i * (kb + 4.0)
     if name == "sort":
-        # tile sort: one histogram read of the ids, per pass a read and a write of (id, emit position); the
-        # first pass takes the positions from the key index instead of reading them
+        # tile sort: one read of the ids for the digit counts (the later passes' are not counted), per pass a read and a
+        # write of (id, emit position); the first pass takes the positions from the key index instead of reading them
         return i * (kb + 2.0 * (kb + 4.0) * shape["tile_passes"] - 4.0)
     if name == "offsets":
         return 4.0 * (px / 256.0)

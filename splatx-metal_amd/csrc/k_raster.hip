@@ -2,7 +2,8 @@
 //
 // Contracts: rasterize_to_pixels_3dgs_fwd/bwd (Rasterize3DGSFwd.metal:57-204,
 // Rasterize3DGSBwd.metal:70-298). One 256-thread workgroup (4 waves of 64) per 16x16 tile, one
-// thread per pixel. Splat records (3 x float4) are staged through LDS in batches of 256.
+// thread per pixel, except the forward of images of up to kWideTiles tiles (k_raster_fwd_wide: 1024 threads, a wave per
+// block). Splat records (3 x float4) are staged through LDS in batches of 256 (wide: 512).
 //
 // Block groups: the tile is sixteen 4x4 pixel blocks. Wave w covers the 8x8 quadrant
 // (w & 1, w >> 1); its lanes form four 16-lane groups, one block each (lane l: group l >> 4, pixel
@@ -1331,8 +1332,12 @@ void raster_tile_order(const int32_t* offsets, int n_tiles, int64_t n_isects, in
 
 // Up to this many tiles a tile gets a wave per block: the GPU holds two such workgroups per compute unit (64 VGPRs),
 // so all of them run at once. Measured, four waves a tile and sixteen: 260 tiles of 2 thousand entries 121 and 73 us,
-// of 4 thousand 258 and 145, 256 tiles of 200 entries 26 and 17, 512 tiles of large splats (every block reached) 39
-// and 41; past 512, where a second round begins, 544 tiles of large splats 40 and 48.
+// of 4 thousand 258 and 145. Up to 256 tiles sixteen are faster throughout (256 tiles of 50 entries 16.4 and 14.3, of
+// 230 48 and 32, of large splats 31 to 44 and 24 to 30). From 257 to 512, where compute units hold two, it depends on
+// the list: 512 tiles of 270 entries 51 and 37, of 170 27.5 and 20.8, of 56 18.2 and 18.1; of large splats that reach
+// every block and soon hide the rest 37 to 39 and 37 to 40, at 416 to 512 tiles up to 2.4 us more with sixteen. The
+// list's kind is not known on the host, and the gain is the larger side. Past 512, where a second round begins, 528 tiles of
+// large splats 38 to 40 and 44 to 47.
 constexpr int kWideTiles = 512;
 
 void raster_fwd(const RasterArgs& a, float* rgb, float* alpha, int32_t* last, hipStream_t s) {

@@ -96,7 +96,8 @@ struct sxh_executor {
     hipGraphExec_t graph_b[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     bool use_graph = true;
     // test switch (environment SXH_DEBUG_FORCE_SORT_ERROR=1 at creation): after the tile sort, a kernel
-    // sets the sort's error word, as a sort that gave up would; every kernel still runs to its end
+    // sets the sort's error word (no sort does; the update, the host and the readback heed it as a guard); every kernel
+    // still runs to its end
     bool debug_sort_error = false;
     int isect_order = SXH_ISECT_ORDER_AUTO;
     // The last training step's parameter update is deferred: the next training step applies it in its

@@ -5,7 +5,7 @@
 // 43 ms), where the link moves 56 GB/s, one thread's memcpy 29 GB/s and four threads' 56 GB/s; and 18 copies of
 // a few kB each cost 0.5 ms. Here the chunks of a whole list of arrays run through one ring: neighbouring
 // arrays share chunks, and a few threads copy between the caller's memory and the pinned chunks while the link
-// moves others.
+// moves others: the 708 MB take 18.3 ms to the device and 16 back.
 #pragma once
 
 #include <hip/hip_runtime.h>
